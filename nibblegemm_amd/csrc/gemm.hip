@@ -4,10 +4,10 @@
 // checks :379-429).  The reference decodes B into shared memory and feeds
 // wmma / mma.sync; here the tile feeds v_mfma_f32_32x32x16_f16.
 //
-// Two kernels share the tile arithmetic.  gemm_pc64_kernel (further down)
-// runs wherever its 16-byte B loads apply: four waves multiply while four
-// others load and decode the next 64-k step.  gemm_tile_kernel, described
-// here, serves the remaining operands (N % 4 != 0, under-aligned weights).
+// Three kernels.  The direct kernel (gemm_direct.h) runs nearly everything;
+// gemm_pc64_kernel (further down) short batches over a middling K with few
+// tiles; gemm_tile_kernel, described here, the operands neither takes (odd N,
+// weights or scales not aligned for loads of two columns).
 //
 // Tile: BM x BN x 32 per workgroup of 4 wave64s (2 x 2), each wave owning a
 // (BM/2) x (BN/2) block of 32 x 32 MFMA tiles.  Per 32-k step:
@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "gemm_direct.h"
 #include "nibble_common.h"
 #include "nibble_decode.h"
 #include "stream_matmul.h"
@@ -40,8 +41,6 @@
 namespace nibble {
 
 namespace {
-
-typedef float f16_t __attribute__((ext_vector_type(16)));
 
 constexpr int BK = 32;
 // LDS tile layout.  A tile row (an A row or a B column) holds BK = 32 fp16
@@ -120,10 +119,6 @@ struct BWords<1> {
   static __device__ __forceinline__ uint32_t word(word_t w, int) { return w; }
   static __device__ __forceinline__ _Float16 scale(scale_t x, int) { return x; }
 };
-
-__device__ __forceinline__ f16_t mfma32(h8_t a, h8_t b, f16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
 
 struct TileArgs {
   const _Float16* X;
@@ -436,10 +431,10 @@ gemm_tile_kernel(TileArgs args) {
     __hip_atomic_store(args.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Epilogue of the producer/consumer kernels: the consumer waves hold the
+// Epilogue of the producer/consumer kernel: the consumer waves hold the
 // results (wave block top-left (mw, nw), the tile kernel's register layout);
 // every wave passes the barriers of the K-split exchange.
-template <int TM, int TN, int THREADS, int BM, int BN, bool CAN_SPLIT = true>
+template <int TM, int TN, int THREADS, int BM, int BN>
 __device__ __forceinline__ void pc_epilogue(const f16_t (&acc)[TM][TN], const TileArgs& args,
                                             bool producer, int mw, int nw, int& s_last) {
   const int M = args.M, N = args.N;
@@ -447,8 +442,7 @@ __device__ __forceinline__ void pc_epilogue(const f16_t (&acc)[TM][TN], const Ti
   const int r32 = lane & 31;
   const int rq = (lane >> 5) * 4;
   _Float16* __restrict__ Y = args.Y;
-  // The large-tile kernel never splits K (CAN_SPLIT false): only this path.
-  if (!CAN_SPLIT || args.splits == 1) {
+  if (args.splits == 1) {
     if (producer) return;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -509,32 +503,26 @@ __device__ __forceinline__ int lds_unit64(int r, int c) {
   return 8 * ((r & ~1) | s0) + (c ^ f);
 }
 
-// Producer/consumer form of the tile kernel, with 64-k steps: four producer
-// waves and CWAVES (4 or 8) consumer waves.
+// Producer/consumer form of the tile kernel, with 64-k steps, 64 x 128 tiles:
+// four producer waves and four consumer waves (2 x 2, a 32 x 64 wave tile).
+// It serves short batches over a middling K whose few tiles are split over K
+// (plan_tile): there its narrower tiles make twice the workgroups of the
+// direct kernel's (gemm_direct.h), and the shorter chain of each wins --
+// 129 / 256 x 4096 x 4096 17.3 / 20.5 us against 18.5 / 21.8, 150 x 5120 x
+// 2048 15.0 against 16.5.
 //
-// In the tile kernel above every wave loads, decodes and stores its share of
-// the next step, waits at the barrier and then multiplies, so its MFMA pipe
-// idles while it does the rest (busy about a quarter of a wave's lifetime at
-// M = 2048).  Here the consumer waves only read operands from LDS and issue
-// MFMAs (a 64 x 64 or 32 x 64 wave tile, 16 or 8 MFMAs per wave per step),
-// while the four producer waves run the global-load pipeline and the decode,
-// storing step t + 1 into the other LDS buffer while step t is multiplied.
-// Consumers and producers share the SIMDs, so the decode VALU work and the
-// memory waits overlap the MFMAs.  Both roles pass the same barriers, ntiles
-// + 1 of them, one per step.
-//  * CWAVES = 4 (eight waves, 2 x 2 consumers): BM = 64 or 128; two
-//    workgroups per CU; PSTAGES = 4 steps of loads in flight.
-//  * CWAVES = 8 (twelve waves, 4 x 2 consumers of 64 x 64): BM = 256, one
-//    workgroup per CU (96 KiB of LDS).  Each decoded B tile then serves 256
-//    rows, which halves the decode work and the B stores per FLOP; A's LDS
-//    traffic per FLOP is unchanged.  PSTAGES = 2 (3 and 4 spill or measured
-//    slower, 1 exposes the load latency).
+// The consumer waves only read operands from LDS and issue MFMAs (8 per wave
+// per step), while the producer waves run the global-load pipeline and the
+// decode, storing step t + 1 into the other LDS buffer while step t is
+// multiplied; the decode VALU work and the memory waits overlap the MFMAs.
+// Both roles pass the same barriers, ntiles + 1 of them, one per step.
 //
 // Producers: thread tid loads BM / 32 16-byte A chunks (rows tid / 8 + 32 it,
 // unit tid % 8) and one dwordx4 of B -- packed row tid / 32 of the step,
-// columns 4 (tid % 32) .. + 3 -- with its four scales.  BN = 128.
-template <int BM, int GROUP, int CWAVES = 4, int PSTAGES = kStages>
-__global__ __launch_bounds__((CWAVES + 4) * 64) void gemm_pc64_kernel(TileArgs args) {
+// columns 4 (tid % 32) .. + 3 -- with its four scales.
+template <int GROUP>
+__global__ __launch_bounds__(8 * 64) void gemm_pc64_kernel(TileArgs args) {
+  constexpr int BM = 64, CWAVES = 4, PSTAGES = kStages;
   constexpr int BN = 128;
   constexpr int PBK = 64;
   constexpr int THREADS = (CWAVES + 4) * 64;
@@ -542,8 +530,6 @@ __global__ __launch_bounds__((CWAVES + 4) * 64) void gemm_pc64_kernel(TileArgs a
   constexpr int WM = BM / WROWS, WN = BN / 2;
   constexpr int TM = WM / 32, TN = WN / 32;          // 32 x 32 MFMA tiles per wave
   constexpr int A_IT = BM * (PBK / 8) / kGemmThreads;
-  static_assert(CWAVES == 4 || CWAVES == 8, "four or eight consumer waves");
-  static_assert(TM >= 1 && PSTAGES >= 1 && PSTAGES <= 4, "wave tile and load ring");
   __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * PBK];
   __shared__ __attribute__((aligned(16))) _Float16 Bs[2][BN * PBK];
   __shared__ int s_last;
@@ -634,26 +620,20 @@ __global__ __launch_bounds__((CWAVES + 4) * 64) void gemm_pc64_kernel(TileArgs a
       __syncthreads();
     };
     using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, (PSTAGES > 1 ? 1 : 0)>;
-    using I2 = std::integral_constant<int, (PSTAGES > 2 ? 2 : 0)>;
-    using I3 = std::integral_constant<int, (PSTAGES > 3 ? 3 : 0)>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
     int i = 0;
     for (; i + PSTAGES <= ntiles; i += PSTAGES) {
       piter(I0{}, i);
-      if constexpr (PSTAGES > 1) piter(I1{}, i + 1);
-      if constexpr (PSTAGES > 2) piter(I2{}, i + 2);
-      if constexpr (PSTAGES > 3) piter(I3{}, i + 3);
+      piter(I1{}, i + 1);
+      piter(I2{}, i + 2);
+      piter(I3{}, i + 3);
     }
     const int rem = ntiles - i;  // < PSTAGES
-    if constexpr (PSTAGES > 1) {
-      if (rem > 0) piter(I0{}, i);
-    }
-    if constexpr (PSTAGES > 2) {
-      if (rem > 1) piter(I1{}, i + 1);
-    }
-    if constexpr (PSTAGES > 3) {
-      if (rem > 2) piter(I2{}, i + 2);
-    }
+    if (rem > 0) piter(I0{}, i);
+    if (rem > 1) piter(I1{}, i + 1);
+    if (rem > 2) piter(I2{}, i + 2);
     __syncthreads();
   } else {
     int rda[TM][PBK / 16], rdb[TN][PBK / 16];
@@ -682,213 +662,30 @@ __global__ __launch_bounds__((CWAVES + 4) * 64) void gemm_pc64_kernel(TileArgs a
       __syncthreads();
     }
   }
-  // The twelve-wave form is planned without a K split.
-  pc_epilogue<TM, TN, THREADS, BM, BN, CWAVES == 4>(acc, args, producer, m0 + wm, n0 + wn, s_last);
+  pc_epilogue<TM, TN, THREADS, BM, BN>(acc, args, producer, m0 + wm, n0 + wn, s_last);
 }
 
-template <int BM>
 hipError_t launch_pc64(const TileArgs& a, int64_t G, hipStream_t stream) {
-  dim3 grid(static_cast<unsigned>(ceil_div(a.N, 128)), static_cast<unsigned>(ceil_div(a.M, BM)),
+  dim3 grid(static_cast<unsigned>(ceil_div(a.N, 128)), static_cast<unsigned>(ceil_div(a.M, 64)),
             static_cast<unsigned>(a.splits));
   if (G == 128)
-    gemm_pc64_kernel<BM, 128><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
+    gemm_pc64_kernel<128><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
   else
-    gemm_pc64_kernel<BM, 64><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
+    gemm_pc64_kernel<64><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
   return hipGetLastError();
 }
 
-// 256-row tiles, eight consumer waves; never split over K.
-hipError_t launch_pc256(const TileArgs& a, int64_t G, hipStream_t stream) {
-  if (a.splits != 1) return hipErrorInvalidValue;
-  dim3 grid(static_cast<unsigned>(ceil_div(a.N, 128)), static_cast<unsigned>(ceil_div(a.M, 256)), 1);
+template <int TM, int KW>
+hipError_t launch_direct_cfg(const DirectArgs& a, int64_t G, hipStream_t stream) {
+  // Up to 4 row tiles a wave leaves registers for two waves per SIMD.
+  constexpr int kOcc = TM <= 4 ? 2 : 1;
+  const unsigned grid = static_cast<unsigned>(a.tiles_m) * a.tiles_n * a.splits;
   if (G == 128)
-    gemm_pc64_kernel<256, 128, 8, 2><<<grid, 12 * 64, 0, stream>>>(a);
+    gemm_direct_kernel<TM, KW, 128, kOcc><<<grid, KW * kDirectWaves * 64, 0, stream>>>(a);
   else
-    gemm_pc64_kernel<256, 64, 8, 2><<<grid, 12 * 64, 0, stream>>>(a);
+    gemm_direct_kernel<TM, KW, 64, kOcc><<<grid, KW * kDirectWaves * 64, 0, stream>>>(a);
   return hipGetLastError();
 }
-
-// Large-tile form for big batches: 256 x 256 output tiles, four waves (one
-// per SIMD), each wave a (BM/2) x (BN/2) block of 32 x 32 MFMA tiles held in
-// registers (256 accumulators per lane).  Every wave loads, decodes, stores
-// and multiplies, like the tile kernel, but an operand read from LDS now
-// feeds four MFMAs instead of two, halving the LDS traffic per FLOP of the
-// 128 x 128 producer/consumer kernel.  64-k steps, LDS double buffered
-// (2 x 64 KiB), global loads two steps ahead in registers, one barrier per
-// step.  The template also builds 256 x 128 and 128 x 256 tiles; measured on
-// MI355X they lost to the 128 x 128 producer/consumer kernel wherever they
-// were the largest tile to fill the chip (14336 x 4096, M = 2048: 267 and
-// 250 us against 242 us), so the planner does not use them.
-//
-// Loads per thread and step: BM / 32 16-byte A chunks (rows tid / 8 + 32 it,
-// unit tid % 8) and BN / 128 dwordx4 of packed B (columns 4 q .. 4 q + 3,
-// q = tid % (BN / 4), packed rows tid / (BN / 4) apart by 256 / (BN / 4))
-// with their four scales.
-template <int BM, int BN, int GROUP>
-__global__ __launch_bounds__(kGemmThreads) void gemm_big_kernel(TileArgs args) {
-  constexpr int PBK = 64;
-  constexpr int TM = BM / 64, TN = BN / 64;                   // 32 x 32 tiles per wave
-  constexpr int A_IT = BM * (PBK / 8) / kGemmThreads;          // 16-byte A chunks per thread
-  constexpr int QUADS = BN / 4;                                // column quads per packed row
-  constexpr int B_IT = (PBK / 8) * QUADS / kGemmThreads;       // packed quads per thread
-  constexpr int PR_STEP = kGemmThreads / QUADS;                // packed rows apart
-  static_assert(GROUP % PBK == 0, "one scale per column per step");
-  static_assert(B_IT >= 1 && A_IT >= 1, "tile too small for the loaders");
-  __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * PBK];
-  __shared__ __attribute__((aligned(16))) _Float16 Bs[2][BN * PBK];
-  __shared__ int s_last;
-  const int M = args.M, K = args.K, N = args.N;
-  const int tid = static_cast<int>(threadIdx.x);
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
-  const int step0 = blockIdx.z * args.steps_per_split;
-  const int ntiles = min(args.steps_per_split, K / PBK - step0);
-  const int wm = (wave >> 1) * (BM / 2);
-  const int wn = (wave & 1) * (BN / 2);
-  const int r32 = lane & 31;
-
-  struct Stage {
-    h8_t a[A_IT];
-    u4_t b[B_IT];
-    h4_t s;
-  };
-  const uint32_t row_bytes = args.L.w_row;
-  const __amdgpu_buffer_rsrc_t rx =
-      make_rsrc(args.X, static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 2u);
-  const __amdgpu_buffer_rsrc_t rw =
-      make_rsrc(args.Wq, static_cast<uint32_t>(K / 8) * static_cast<uint32_t>(N) * 4u);
-  const __amdgpu_buffer_rsrc_t rsc =
-      make_rsrc(args.S, static_cast<uint32_t>(K / GROUP) * static_cast<uint32_t>(N) * 2u);
-  uint32_t voff_a[A_IT];
-  int a_st[A_IT];
-#pragma unroll
-  for (int it = 0; it < A_IT; ++it) {
-    const int row = (tid >> 3) + 32 * it;
-    const int gm = m0 + row;
-    voff_a[it] = gm < M ? (static_cast<uint32_t>(gm) * K + (tid & 7) * 8) * 2u : kOutOfRange;
-    a_st[it] = lds_unit64(row, tid & 7) * 8;
-  }
-  const int quad = tid % QUADS;
-  const int b_col = n0 + 4 * quad;
-  const bool b_ok = b_col < N;  // N % 4 == 0: the quad is wholly inside or outside
-  uint32_t voff_b[B_IT];
-  int b_st[B_IT][4];
-#pragma unroll
-  for (int it = 0; it < B_IT; ++it) {
-    const int pr = tid / QUADS + PR_STEP * it;
-    voff_b[it] = b_ok ? pr * row_bytes + args.L.wcol(b_col) : kOutOfRange;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b_st[it][j] = lds_unit64(4 * quad + j, pr) * 8;
-  }
-  const uint32_t voff_s = b_ok ? args.L.scol(b_col) : kOutOfRange;
-
-  auto load_step = [&](Stage& st, int step) {
-    const uint32_t k0 = static_cast<uint32_t>((step0 + min(step, ntiles - 1)) * PBK);
-#pragma unroll
-    for (int it = 0; it < A_IT; ++it)
-      st.a[it] = __builtin_bit_cast(
-          h8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, voff_a[it], k0 * 2u, 0));
-#pragma unroll
-    for (int it = 0; it < B_IT; ++it)
-      st.b[it] = __builtin_bit_cast(
-          u4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, voff_b[it], (k0 / 8) * row_bytes, 0));
-    st.s = __builtin_bit_cast(
-        h4_t, __builtin_amdgcn_raw_buffer_load_b64(
-                  rsc, voff_s, (k0 / GROUP) * args.L.s_row, 0));
-  };
-  auto store_step = [&](const Stage& st, int buf) {
-#pragma unroll
-    for (int it = 0; it < A_IT; ++it) *reinterpret_cast<h8_t*>(&As[buf][a_st[it]]) = st.a[it];
-#pragma unroll
-    for (int it = 0; it < B_IT; ++it)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        h2_t w[4];
-        const h2_t s2 = {st.s[j], st.s[j]};
-        decode8_scaled(st.b[it][j], s2, w);
-        const h8_t v = {w[0][0], w[0][1], w[1][0], w[1][1], w[2][0], w[2][1], w[3][0], w[3][1]};
-        *reinterpret_cast<h8_t*>(&Bs[buf][b_st[it][j]]) = v;
-      }
-  };
-
-  f16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  int rda[TM][PBK / 16], rdb[TN][PBK / 16];
-#pragma unroll
-  for (int ks = 0; ks < PBK / 16; ++ks) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) rda[i][ks] = lds_unit64(wm + 32 * i + r32, 2 * ks + (lane >> 5)) * 8;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) rdb[j][ks] = lds_unit64(wn + 32 * j + r32, 2 * ks + (lane >> 5)) * 8;
-  }
-  auto compute_step = [&](int buf) {
-    h8_t a[2][TM], b[2][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) a[0][i] = *reinterpret_cast<const h8_t*>(&As[buf][rda[i][0]]);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) b[0][j] = *reinterpret_cast<const h8_t*>(&Bs[buf][rdb[j][0]]);
-#pragma unroll
-    for (int ks = 0; ks < PBK / 16; ++ks) {
-      const int cur = ks & 1;
-      if (ks + 1 < PBK / 16) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          a[cur ^ 1][i] = *reinterpret_cast<const h8_t*>(&As[buf][rda[i][ks + 1]]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          b[cur ^ 1][j] = *reinterpret_cast<const h8_t*>(&Bs[buf][rdb[j][ks + 1]]);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(a[cur][i], b[cur][j], acc[i][j]);
-    }
-  };
-
-  Stage R0, R1;
-  load_step(R0, 0);
-  load_step(R1, 1);
-  store_step(R0, 0);
-  load_step(R0, 2);
-  __syncthreads();
-  int t = 0;
-  for (; t + 2 <= ntiles; t += 2) {
-    compute_step(0);
-    store_step(R1, 1);
-    load_step(R1, t + 3);
-    __syncthreads();
-    compute_step(1);
-    store_step(R0, 0);
-    load_step(R0, t + 4);
-    __syncthreads();
-  }
-  if (t < ntiles) {
-    compute_step(0);
-    __syncthreads();
-  }
-  pc_epilogue<TM, TN, kGemmThreads, BM, BN, false>(acc, args, false, m0 + wm, n0 + wn, s_last);
-}
-
-template <int BM, int BN>
-hipError_t launch_big(const TileArgs& a, int64_t G, hipStream_t stream) {
-  if (a.splits != 1) return hipErrorInvalidValue;  // the kernel sums all of K
-  dim3 grid(static_cast<unsigned>(ceil_div(a.N, BN)), static_cast<unsigned>(ceil_div(a.M, BM)),
-            static_cast<unsigned>(a.splits));
-  if (G == 128)
-    gemm_big_kernel<BM, BN, 128><<<grid, kGemmThreads, 0, stream>>>(a);
-  else
-    gemm_big_kernel<BM, BN, 64><<<grid, kGemmThreads, 0, stream>>>(a);
-  return hipGetLastError();
-}
-
 
 template <int BM, int BN>
 hipError_t launch_tile(const TileArgs& a, int64_t G, hipStream_t stream) {
@@ -901,36 +698,25 @@ hipError_t launch_tile(const TileArgs& a, int64_t G, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Which kernel a call runs, and its tile: the direct kernel's (tm > 0: 32 tm
+// rows by 256 columns, kw teams), the producer/consumer kernel's 64 x 128, or
+// the tile kernel's bm x bn.
 struct TileChoice {
   int bm, bn;
-  bool pc = false;   // the producer/consumer kernel (BN = 128, 64-k steps)
-  bool big = false;  // the 256 x 256 large-tile kernel (64-k steps)
+  bool pc = false;
+  int tm = 0, kw = 1;
 };
-
-// Batches from this many rows up may run the twelve-wave producer/consumer
-// kernel (256 x 128 tiles, version 6).
-constexpr int64_t kPc256MinM = 2048;
 
 // The device the plans are made for: MI355X, 256 CUs.  Planning with a fixed
 // count keeps the workspace query pure host code and equal to the launch.
 constexpr int kPlanCUs = 256;
-
-// A grid of one-workgroup-per-CU tiles that fills whole rounds of the CUs,
-// the last at least 7/8 full.
-bool whole_rounds(int64_t tiles) {
-  const int64_t last = tiles % kPlanCUs;
-  return tiles >= kPlanCUs && (last == 0 || 8 * last >= 7 * kPlanCUs);
-}
-
-// Batches from this many rows up may run the large-tile kernel (version 6).
-constexpr int64_t kBigMinM = 1024;
 
 // The widest B vector aligned operands of this N allow (the plan the
 // workspace query assumes).
 int nominal_bn_max(int64_t N) { return N % 4 == 0 ? 256 : N % 2 == 0 ? 128 : 64; }
 
 // k per pipeline step of the kernel a choice runs.
-int step_k(TileChoice t) { return t.pc || t.big ? 64 : BK; }
+int step_k(TileChoice t) { return t.pc || t.tm > 0 ? 64 : BK; }
 
 // Widest B vector (BN / 64 packed words per thread) the operands allow.
 int max_bn(int64_t N, const void* w, const void* s) {
@@ -953,12 +739,6 @@ TileChoice choose_tile(int64_t M, int64_t N, int bn_max) {
   return {64, bn};
 }
 
-// Launch plan of the tile kernel.  Long reductions (K >= 8192) with few
-// output tiles split K so the grid reaches two workgroups per CU, at most 4
-// ways.  Measured at 14336 x 4096 (64 x 128 tiles): M = 128 from 126 us to
-// 70 us (4 splits), M = 512 from 129 us to 117 us (2 splits).  At K = 4096
-// every split measured slower: the partial round trip outweighs the extra
-// parallelism.
 struct TilePlan {
   TileChoice t;
   int splits = 1;
@@ -967,66 +747,27 @@ struct TilePlan {
   size_t workspace_bytes = 0;
 };
 
-TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max) {
+// The K splits a shape may use and the workspace they need -- what the
+// workspace query answers, so what a caller's buffer holds -- with the tile
+// that runs where the direct kernel does not.  Long reductions split where
+// the tiles are few, as does 4096 <= K < 8192 with at most 160 64-row tiles.
+// The direct kernel takes as many of these splits as pay (plan_tile).
+TilePlan plan_split_room(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max) {
   TilePlan p;
   int64_t tiles = 0;
   int splits = 1;
-  // 256 x 256 tiles when the grid is one round over the CUs, at least 7/8
-  // full; never split over K.  Measured on MI355X against the 128 x 128
-  // producer/consumer kernel, graph replays interleaved with each other and
-  // with hipBLASLt: 1024 x 4096 x 14336 (224 tiles) 128 vs 133 us,
-  // 4096 x 14336 x 4096 (256 tiles) 414 vs 464 us.  Grids of several rounds
-  // lost under that load: 2048 and 4096 x 4096 x 14336 (448 and 896 tiles,
-  // 1.75 and 3.5 rounds) 254 vs 242 and 495 vs 474 us.  Their last round is
-  // part-empty, and with one workgroup per CU no other workgroup's MFMAs
-  // overlap a tile's prologue and epilogue.
-  const int64_t t256 = ceil_div(M, 256) * ceil_div(N, 256);
-  const bool big = version == 6 && M >= kBigMinM && K % 64 == 0 && bn_max >= 256 &&
-                   8 * t256 >= 7 * kPlanCUs && t256 <= kPlanCUs;
   if (M <= kStreamMaxM && K % 64 == 0 && bn_max >= 256) {
-    // Small batches that do not stream (gemm_streams): 64-row tiles of the
-    // producer/consumer kernel, K split so that the grid nears one round of
-    // the CUs -- the largest of 1, 2, 4, 8 ways keeping it within 320
-    // workgroups.  Both versions take this plan (so they agree to the bit).
+    // Small batches that do not stream (gemm_streams): the largest of 1, 2, 4,
+    // 8 ways keeping the grid of 64-row tiles within 320 workgroups.  Both
+    // versions take this plan (so they agree to the bit).
     p.t = TileChoice{64, 128, true};
     tiles = ceil_div(M, 64) * ceil_div(N, 128);
     while (splits < 8 && tiles * splits * 2 <= 320 && K / 64 >= 2 * splits) splits *= 2;
-  } else if (big) {
-    p.t = TileChoice{256, 256, false, true};
-    tiles = t256;
-  } else if (version == 6 && M >= kPc256MinM && K % 64 == 0 && bn_max >= 256 &&
-             whole_rounds(ceil_div(M, 256) * ceil_div(N, 128))) {
-    // 256 x 128 tiles with eight consumer waves, one workgroup per CU, where
-    // their grid makes whole rounds of the CUs (the last at least 7/8 full);
-    // never split over K.  Measured on MI355X against the 128 x 128 kernel
-    // (graph replays interleaved with hipBLASLt): 2048 x 14336 x 4096 (256
-    // tiles, one round) 232 vs 245 us; 4096 x 4096 x 14336 (1792 tiles,
-    // seven rounds) 470 vs 491.  With a part-filled last round the 128 x 128
-    // kernel's two workgroups per CU balance better: 2048 and 3072 x 4096 x
-    // 14336 (3.5 and 5.25 rounds) 254 vs 248 and 385 vs 378, 3072 x 14336 x
-    // 4096 (1.5 rounds) 405 vs 365.
-    p.t = TileChoice{256, 128, true};
-    tiles = ceil_div(M, 256) * ceil_div(N, 128);
   } else if (K % 64 == 0 && bn_max >= 256) {
-    // The producer/consumer kernel wherever it applies (whole 64-k steps,
-    // 16-byte packed-word loads).  Measured on MI355X, graph replay:
-    //  * K < 8192 (no split): 128-row tiles once the launch has ~192 of them
-    //    (4096 x 14336 from M = 160), 64-row tiles below;
-    //  * K >= 8192: 128-row tiles, split over K by the tile count -- at
-    //    14336 x 4096, M = 160 (64 tiles) 4 ways: 41 us (64-row tiles,
-    //    2 ways: 58); M = 384 / 512 (96 / 128 tiles) 2 ways: 74 / 76 us
-    //    (97 / 101); M = 768 / 1024 (192 / 256 tiles) unsplit; M = 1536
-    //    (384 tiles, a round and a half) 2 ways: 202 us (242 unsplit);
-    //    M = 2048 (512 tiles) unsplit.  The split's partials are summed by
-    //    the whole last workgroup of each tile (tile_sum_splits);
-    //  * 4096 <= K < 8192 with at most 160 64-row tiles: 4 ways -- 4096 x
-    //    4096, M = 129 / 192 / 256 (96 / 96 / 128 tiles) 16.7 / 17.4 /
-    //    19.3 us unsplit 25.0 / 25.3 / 25.0; 4096 x 6144, M = 129 / 160 /
-    //    192 (144 tiles) 21.2 / 22.5 / 23.7 unsplit 25.6 / 25.3 / 25.0; at
-    //    192 tiles (4096 x 6144, M = 256) unsplit is ahead, 25.5 vs 27.4.
     const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
-    p.t = TileChoice{version == 7 || K >= 8192 || t128 >= 192 ? 128 : 64, 128, true};
-    tiles = ceil_div(M, p.t.bm) * ceil_div(N, 128);
+    const int bm = version == 7 || K >= 8192 || t128 >= 192 ? 128 : 64;
+    p.t = TileChoice{bm, 128, bm == 64};
+    tiles = ceil_div(M, bm) * ceil_div(N, 128);
     if (K >= 8192) {
       if (tiles <= 64)
         splits = 4;
@@ -1034,7 +775,7 @@ TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max)
         splits = 2;
       else if (tiles > kPlanCUs && tiles < 2 * kPlanCUs)
         splits = 2;
-    } else if (p.t.bm == 64 && K >= 4096 && tiles <= 160) {
+    } else if (bm == 64 && K >= 4096 && tiles <= 160) {
       splits = 4;
     }
   } else {
@@ -1053,14 +794,102 @@ TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max)
   return p;
 }
 
+// Widest N the direct kernel addresses: a tile's rows within 32-bit offsets.
+constexpr int64_t kDirectMaxN = int64_t(1) << 22;
+
+// Whether the direct kernel takes these operands: two columns a load.
+bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
+  return K % 64 == 0 && N % 2 == 0 && N < kDirectMaxN && aligned(w, 8) && aligned(s, 4);
+}
+
+// The direct kernel's tile, teams and splits for a shape, within the splits
+// and counters of `room`.  A model of its time, fitted to MI355X measurements
+// of every tile at some 30 shapes (M = 33..4096), us: 4.5 to start and drain;
+// per 64-k step and round of the CUs the tile's own time when few workgroups
+// run, kStep; 0.36 of the time the whole product takes at the power-limited
+// 1.25 PFLOP/s; and for a K split 3 plus its partials at 2.5 TB/s.  Tiles of
+// up to 4 row tiles share a CU two at a time, so their last round is half as
+// dear.  It names the fastest tile or one within ~5% at nearly all of them:
+// e.g. 512 x 4096 x 14336 tm = 4 55 us (3: 69, 8: 75), 1000 x 5504 x 4102
+// tm = 3 50 (4: 55), 256 x 4096 x 14336 tm = 2 33 (4: 40, 8: 72), 3000 x
+// 3072 x 3008 tm = 5 54 (3: 57, 4: 66), 129 x 14336 x 4096 tm = 2, 4 splits
+// 32 (unsplit 77), 4096 x 4096 x 4096 tm = 8 108 (4: 111).
+// Up to 96 rows a tile, two teams halve a long K within the workgroup; K <
+// 2048 is too short for that to pay.
+TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, int* splits) {
+  struct Cfg {
+    int tm;
+    double step, step2;  // one team, two teams
+  };
+  static constexpr Cfg kCfgs[] = {{1, 0.36, 0.28}, {2, 0.40, 0.36}, {3, 0.45, 0.40},
+                                  {4, 0.53, 0.0},  {5, 0.68, 0.0},  {6, 0.80, 0.0},
+                                  {8, 1.03, 0.0}};
+  const int64_t tiles_n = ceil_div(N, kDirectBN), steps = K / kDirectStep;
+  const int64_t max_counters = static_cast<int64_t>(room.counter_bytes / 4);
+  const double power = 0.36 * 2.0 * static_cast<double>(M) * K * N / 1.25e9;
+  TileChoice best{0, kDirectBN};
+  double best_us = 1e30;
+  for (const Cfg& c : kCfgs) {
+    const bool teams = c.step2 > 0 && K >= 2048;
+    const double step = teams ? c.step2 : c.step;
+    const int64_t tiles = ceil_div(M, 32 * c.tm) * tiles_n;
+    for (int s = 1; s <= (c.tm <= kDirectMaxSplitTM ? room.splits : 1); ++s) {
+      if (s > 1 && tiles > max_counters) break;
+      const int64_t per = ceil_div(steps, s);
+      if (ceil_div(steps, per) != s) continue;  // not a split count that divides evenly enough
+      const double fill = static_cast<double>(tiles * s) / kPlanCUs;
+      const double rounds = static_cast<double>(ceil_div(tiles * s, kPlanCUs));
+      const double eff = c.tm <= 4 && fill > 1 ? 0.5 * (rounds + fill) : rounds;
+      double us = 4.5 + eff * static_cast<double>(per) * step + power;
+      if (s > 1) us += 3.0 + static_cast<double>(s) * M * N * 4 / 2.5e6;
+      if (us < best_us) {
+        best_us = us;
+        best.bm = 32 * c.tm;
+        best.tm = c.tm;
+        best.kw = teams ? 2 : 1;
+        *splits = s;
+      }
+    }
+  }
+  return best;
+}
+
+// The launch plan.  `direct` says the operands suit the direct kernel.  Both
+// versions take the same plan wherever their workspaces agree, so they agree
+// to the bit.
+TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max, bool direct) {
+  TilePlan p = plan_split_room(M, K, N, version, bn_max);
+  // The 64 x 128 tiles keep the mid-K shapes they are split 4 ways for.
+  const bool mid_k = M > kStreamMaxM && p.t.pc && p.splits > 1;
+  if (direct && !mid_k) {
+    int splits = 1;
+    p.t = choose_direct(M, K, N, p, &splits);
+    p.splits = splits;
+    p.steps_per_split = static_cast<int>(ceil_div(K / kDirectStep, splits));
+  }
+  return p;
+}
+
+hipError_t launch_direct(TileChoice t, DirectArgs a, int64_t G, hipStream_t stream) {
+  a.tiles_m = static_cast<int>(ceil_div(a.M, 32 * t.tm));
+  a.tiles_n = static_cast<int>(ceil_div(a.N, kDirectBN));
+  switch (t.tm * 2 + t.kw - 1) {
+    case 2: return launch_direct_cfg<1, 1>(a, G, stream);
+    case 3: return launch_direct_cfg<1, 2>(a, G, stream);
+    case 4: return launch_direct_cfg<2, 1>(a, G, stream);
+    case 5: return launch_direct_cfg<2, 2>(a, G, stream);
+    case 6: return launch_direct_cfg<3, 1>(a, G, stream);
+    case 7: return launch_direct_cfg<3, 2>(a, G, stream);
+    case 8: return launch_direct_cfg<4, 1>(a, G, stream);
+    case 10: return launch_direct_cfg<5, 1>(a, G, stream);
+    case 12: return launch_direct_cfg<6, 1>(a, G, stream);
+    case 16: return launch_direct_cfg<8, 1>(a, G, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 hipError_t launch_choice(TileChoice t, const TileArgs& a, int64_t G, hipStream_t stream) {
-  if (t.big) {
-    return launch_big<256, 256>(a, G, stream);
-  }
-  if (t.pc) {
-    if (t.bm == 256) return launch_pc256(a, G, stream);
-    return t.bm == 128 ? launch_pc64<128>(a, G, stream) : launch_pc64<64>(a, G, stream);
-  }
+  if (t.pc) return launch_pc64(a, G, stream);
   if (t.bm == 128 && t.bn == 128) return launch_tile<128, 128>(a, G, stream);
   if (t.bm == 64 && t.bn == 128) return launch_tile<64, 128>(a, G, stream);
   if (t.bm == 128 && t.bn == 64) return launch_tile<128, 64>(a, G, stream);
@@ -1146,7 +975,7 @@ void gemm_plan_bytes(int64_t M, int64_t K, int64_t N, int64_t G, int64_t version
     *counters = p.counter_bytes;
     return;
   }
-  const TilePlan p = plan_tile(M, K, N, version, nominal_bn_max(N));
+  const TilePlan p = plan_split_room(M, K, N, version, nominal_bn_max(N));
   *ws = p.workspace_bytes;
   *counters = p.counter_bytes;
 }
@@ -1182,7 +1011,8 @@ namespace {
 // bits.
 int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, const void* S,
              int64_t group_size, int64_t version, void* Y, void* workspace,
-             size_t workspace_bytes, void* stream_, int64_t strip_cols) {
+             size_t workspace_bytes, void* stream_, int64_t strip_cols, int epilogue = 0,
+             const void* bias = nullptr) {
   int rc = NIBBLE_OK;
   if (M == 0 || N == 0) return ok();
   hipStream_t stream = static_cast<hipStream_t>(stream_);
@@ -1193,7 +1023,8 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
     NIBBLE_HIP(fill_zero_f16(Y, M * N, stream));
     return ok();
   }
-  if (gemm_streams(M, K, N, group_size) && stream_supported(X, Wq, S, Y, M, K, N, group_size)) {
+  if (epilogue == kEpilogueNone && gemm_streams(M, K, N, group_size) &&
+      stream_supported(X, Wq, S, Y, M, K, N, group_size)) {
     StreamPlan p;
     rc = plan_stream(M, K, N, group_size, true, 0, 0, &p);
     if (rc != NIBBLE_OK) return rc;
@@ -1203,11 +1034,13 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
   }
   const auto* x = static_cast<const _Float16*>(X);
   auto* y = static_cast<_Float16*>(Y);
-  // Version 6 picks the tile for the shape; version 7 runs 128-row tiles.
-  // Every tile accumulates each output over k in the same order, so without
-  // a K split the two give identical bits (as the reference's v6 and v7 do).
+  // The tiles sum every output over k in the same order, so without a K split
+  // (or two teams) they give identical bits.
   const int bn_max = max_bn(N, Wq, S);
-  TilePlan p = plan_tile(M, K, N, version, bn_max);
+  const bool direct = direct_supported(K, N, Wq, S);
+  TilePlan p = plan_tile(M, K, N, version, bn_max, direct);
+  if (epilogue != kEpilogueNone && p.t.tm == 0)
+    return fail(NIBBLE_ERR_UNSUPPORTED, "no fused epilogue for this shape (nibble_gemm_fuses)");
   // The kernel addresses X through a buffer resource with 32-bit offsets:
   // tall activations are run in row blocks that stay below 2^31 bytes (such
   // grids are far too large to need a K split).
@@ -1216,9 +1049,13 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
   // another kernel than that plan's (tiles where the query planned the
   // streaming kernel, or another tile), the call runs without a split, as do
   // row-blocked tall launches.
-  const TilePlan nominal = plan_tile(M, K, N, version, nominal_bn_max(N));
+  const bool nominal_direct = direct_supported(K, N, nullptr, nullptr);
+  const TilePlan nominal = bn_max == nominal_bn_max(N) && direct == nominal_direct
+                               ? p
+                               : plan_tile(M, K, N, version, nominal_bn_max(N), nominal_direct);
   if (M > rows_max || gemm_streams(M, K, N, group_size) || p.t.pc != nominal.t.pc ||
-      p.t.big != nominal.t.big || p.t.bm != nominal.t.bm || p.t.bn != nominal.t.bn)
+      p.t.tm != nominal.t.tm || p.t.kw != nominal.t.kw || p.t.bm != nominal.t.bm ||
+      p.t.bn != nominal.t.bn || p.splits != nominal.splits)
     p.splits = 1;
   if (p.splits > 1) {
     if (workspace == nullptr || workspace_bytes < p.workspace_bytes)
@@ -1228,23 +1065,47 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
   } else {
     p.steps_per_split = static_cast<int>(K / step_k(p.t));
   }
-  TileArgs a;
-  a.Wq = static_cast<const uint32_t*>(Wq);
-  a.S = static_cast<const _Float16*>(S);
-  a.K = static_cast<int>(K);
-  a.N = static_cast<int>(N);
-  a.steps_per_split = p.steps_per_split;
-  a.splits = p.splits;
-  a.counters = p.splits > 1 ? static_cast<uint32_t*>(workspace) : nullptr;
-  a.partial = p.splits > 1
-                  ? reinterpret_cast<float*>(static_cast<char*>(workspace) + p.counter_bytes)
-                  : nullptr;
-  a.L = layout_for(K, N, group_size, strip_cols);
+  auto* counters = p.splits > 1 ? static_cast<uint32_t*>(workspace) : nullptr;
+  auto* partial = p.splits > 1
+                      ? reinterpret_cast<float*>(static_cast<char*>(workspace) + p.counter_bytes)
+                      : nullptr;
+  const WeightLayout layout = layout_for(K, N, group_size, strip_cols);
+  const int64_t out_n = epilogue == kEpilogueSwiglu ? N / 2 : N;
   hipError_t e = hipSuccess;
   for (int64_t m0 = 0; m0 < M && e == hipSuccess; m0 += rows_max) {
+    const int rows = static_cast<int>(std::min(rows_max, M - m0));
+    if (p.t.tm > 0) {
+      DirectArgs a{};
+      a.X = x + m0 * K;
+      a.Wq = static_cast<const uint32_t*>(Wq);
+      a.S = static_cast<const _Float16*>(S);
+      a.Y = y + m0 * out_n;
+      a.bias = static_cast<const _Float16*>(bias);
+      a.partial = partial;
+      a.counters = counters;
+      a.M = rows;
+      a.K = static_cast<int>(K);
+      a.N = static_cast<int>(N);
+      a.splits = p.splits;
+      a.steps_per_split = p.steps_per_split;
+      a.epilogue = epilogue;
+      a.L = layout;
+      e = launch_direct(p.t, a, group_size, stream);
+      continue;
+    }
+    TileArgs a;
     a.X = x + m0 * K;
+    a.Wq = static_cast<const uint32_t*>(Wq);
+    a.S = static_cast<const _Float16*>(S);
     a.Y = y + m0 * N;
-    a.M = static_cast<int>(std::min(rows_max, M - m0));
+    a.partial = partial;
+    a.counters = counters;
+    a.M = rows;
+    a.K = static_cast<int>(K);
+    a.N = static_cast<int>(N);
+    a.steps_per_split = p.steps_per_split;
+    a.splits = p.splits;
+    a.L = layout;
     e = launch_choice(p.t, a, group_size, stream);
   }
   if (e != hipSuccess) return hip_fail(e, "gemm kernel launch");

@@ -511,3 +511,41 @@ def test_split_k_sum_into_under_aligned_output():
         assert torch.equal(y, want), start
         assert buf[:start].eq(0).all() and buf[start + M * N:].eq(0).all(), start
         buf.zero_()
+
+
+@pytest.mark.parametrize("K_,g", [(64, 64), (128, 128), (192, 64), (320, 64), (2048, 128), (2176, 64),
+                                  (2240, 64), (2304, 128), (4288, 64)])
+@pytest.mark.parametrize("M,N", [(33, 258), (129, 254), (191, 1030), (256, 512), (700, 514)])
+def test_direct_kernel_edges(M, N, K_, g):
+    """The direct kernel's tails: every remainder of its 4-step rings (one to
+    five 64-k steps, and with two teams from K = 2048 uneven team shares), row
+    tiles and 256-column tiles cut anywhere, N only even, both group sizes.
+    Every output against an fp32 product of the dequant kernel's weights; a
+    step multiplied before its activations had landed would be a whole step
+    off, 1 / sqrt(K / 64) of the rms.  Called 8 times over, the bits repeat."""
+    _, _, _, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
+    ref = Xd.float() @ ng.dequant(qw).float()
+    rms = ref.pow(2).mean().sqrt()
+    ys = [ng.gemm(Xd, qw) for _ in range(8)]
+    torch.cuda.synchronize()
+    assert float((ys[0].float() - ref).abs().max() / rms) <= RMS_TOL
+    for y in ys[1:]:
+        assert torch.equal(y, ys[0])
+
+
+@pytest.mark.parametrize("M,K_,N,g", [(1000, 5504, 4102, 64), (2048, 1344, 6016, 64),
+                                      (1024, 4416, 14336, 64), (3000, 3072, 3008, 128),
+                                      (1536, 14336, 4096, 128), (300, 8256, 1030, 64),
+                                      (66, 8192, 8196, 128)])
+def test_direct_kernel_full_grids(M, K_, N, g):
+    """Grids that fill the CUs (every tile height the plan picks, K splits,
+    K / 64 not a multiple of the ring): every output, and identical bits over
+    20 calls back to back, so no step runs ahead of its copies under load."""
+    _, _, _, Xd, qw = synthetic(M, K_, N, g, seed=M + N)
+    ref = Xd.float() @ ng.dequant(qw).float()
+    rms = ref.pow(2).mean().sqrt()
+    ys = [ng.gemm(Xd, qw) for _ in range(20)]
+    torch.cuda.synchronize()
+    assert float((ys[0].float() - ref).abs().max() / rms) <= RMS_TOL
+    for y in ys[1:]:
+        assert torch.equal(y, ys[0])
