@@ -50,7 +50,7 @@
 extern "C" {
 #endif
 
-#define NIBBLE_ABI_VERSION 14
+#define NIBBLE_ABI_VERSION 15
 
 #if defined(__GNUC__) || defined(__clang__)
 #define NIBBLE_API __attribute__((visibility("default")))
@@ -215,6 +215,18 @@ NIBBLE_API size_t nibble_matmul_fused_workspace_bytes(int64_t M, int64_t K, int6
                                            int64_t group_size, void* stream);
 NIBBLE_API size_t nibble_matmul_fused_counter_bytes(int64_t M, int64_t K, int64_t N,
                                          int64_t group_size, void* stream);
+
+/*
+ * Round-to-nearest quantisation of a dense weight W [K, N] (dtype 0 fp16,
+ * 1 bf16, 2 fp32) into packed words Wq [K/8, N] and fp16 scales S [K/G, N]:
+ * the codes and scales of the reference's quantize
+ * (python/nibblegemm/quant.py:127-161) computed in fp32, a group's scale its
+ * largest magnitude / 7 (at least 1e-8), codes round_half_even(w / scale).
+ * G a multiple of 8 up to 512 (the matmuls take 64 and 128), at most 65535
+ * groups.  The reference quantises on the host; ABI version 15.
+ */
+NIBBLE_API int nibble_quantize_rtn(const void* W, int64_t K, int64_t N, int64_t dtype,
+                        int64_t group_size, void* Wq, void* S, void* stream);
 
 /*
  * Strip-major weights for the decode GEMV (M <= 8).  No counterpart in the

@@ -267,6 +267,19 @@ static PyObject* py_dequant(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
+/* quantize_rtn(W, K, N, dtype, g, Wq, S, stream) */
+static PyObject* py_quantize(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  (void)self;
+  if (!nargs_is(n, 8, "quantize_rtn")) return NULL;
+  void *W, *Wq, *S, *stream;
+  long long K, N, dt, g;
+  if (!take_ptr(a[0], &W) || !take_i64(a[1], &K) || !take_i64(a[2], &N) || !take_i64(a[3], &dt) ||
+      !take_i64(a[4], &g) || !take_ptr(a[5], &Wq) || !take_ptr(a[6], &S) ||
+      !take_ptr(a[7], &stream))
+    return NULL;
+  return PyLong_FromLong(nibble_quantize_rtn(W, K, N, dt, g, Wq, S, stream));
+}
+
 /* gemm_strip_major(X, xr, xc, Wt, St, K, N, g, sw, version, Y, ws, ws_bytes, stream) */
 static PyObject* py_sm_gemm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
@@ -402,6 +415,8 @@ static PyMethodDef kMethods[] = {
      "nibble_pack_strip_major"},
     {"gemv_strip_major", (PyCFunction)(void (*)(void))py_sm_gemv, METH_FASTCALL,
      "nibble_gemv_w4a16_strip_major"},
+    {"quantize_rtn", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL,
+     "nibble_quantize_rtn"},
     {"gemm_strip_major", (PyCFunction)(void (*)(void))py_sm_gemm, METH_FASTCALL,
      "nibble_gemm_w4a16_strip_major"},
     {"dequant_strip_major", (PyCFunction)(void (*)(void))py_sm_dequant, METH_FASTCALL,

@@ -19,8 +19,8 @@ even k take the low four nibbles and the odd k the high four, which is what
 lets the kernels turn two codes sixteen bits apart into one fp16 pair with a
 single mask-and-or.
 
-This module never launches a kernel; :mod:`nibblegemm_amd.ops` never calls its
-host decoders.
+The only kernel this module launches is :func:`quantize_device`'s;
+:mod:`nibblegemm_amd.ops` never calls its host decoders.
 """
 from __future__ import annotations
 
@@ -132,13 +132,51 @@ def quantize(W: torch.Tensor, group_size: int = 128, clip_search: bool = False) 
                            scale.to(torch.float16).cpu().contiguous(), group_size, K, N)
 
 
+#: Weight dtypes the quantisation kernel reads, and its largest group.
+_KERNEL_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
+_KERNEL_MAX_GROUP = 512
+
+
+def _kernel_quantizes(W: torch.Tensor, group_size: int) -> bool:
+    """Whether :func:`quantize_device` runs ``W`` through its kernel: a plain
+    contiguous GPU tensor of a dtype it reads, not one that a tracer, a
+    dispatch mode or a functorch transform wants to see operations on."""
+    return (W.is_cuda and W.dtype in _KERNEL_DTYPES and W.numel() > 0
+            and type(W) in (torch.Tensor, torch.nn.Parameter) and W.is_contiguous()
+            and 8 <= group_size <= _KERNEL_MAX_GROUP and W.shape[0] // group_size < 65536
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 def quantize_device(W: torch.Tensor, group_size: int = 128) -> QuantizedWeight:
     """:func:`quantize` kept on W's device: the same codes, scales and packed
     layout, with ``qweight`` and ``scales`` left where W is (for building large
     weight stacks on the GPU; the reference's ``quantize`` always returns host
-    tensors).  The max-abs scale divides by a tensor of 7s: a GPU divides by a
-    Python scalar as a multiply by its reciprocal, which can round differently
-    from the true division a host ``quantize`` performs."""
+    tensors).  On a GPU one kernel reads W once
+    (``nibble_quantize_rtn``); elsewhere, and for weights the kernel does not
+    read (other dtypes, strided views, groups above 512), the same arithmetic
+    runs as tensor operations."""
+    K, N = _check_quantize_args(W, group_size)
+    if _kernel_quantizes(W, group_size):
+        from . import _native  # noqa: PLC0415  (the host tools need no library)
+        ext = _native.binding()
+        packed = torch.empty((K // PACK_FACTOR, N), dtype=torch.int32, device=W.device)
+        scales = torch.empty((K // group_size, N), dtype=torch.float16, device=W.device)
+        rc = ext.quantize_rtn(W.data_ptr(), K, N, _KERNEL_DTYPES[W.dtype], group_size,
+                              packed.data_ptr(), scales.data_ptr(),
+                              torch.cuda.current_stream(W.device).cuda_stream)
+        if rc:
+            raise RuntimeError(f"nibblegemm_amd: {ext.last_error()} (status {rc})")
+        return QuantizedWeight(packed, scales, group_size, K, N)
+    return _quantize_ops(W, group_size)
+
+
+def _quantize_ops(W: torch.Tensor, group_size: int) -> QuantizedWeight:
+    """:func:`quantize_device` as tensor operations on W's device.  The max-abs
+    scale divides by a tensor of 7s: a GPU divides by a Python scalar as a
+    multiply by its reciprocal, which can round differently from the true
+    division a host ``quantize`` performs."""
     K, N = _check_quantize_args(W, group_size)
     groups = W.detach().float().reshape(K // group_size, group_size, N)
     amax = groups.abs().amax(dim=1)
