@@ -13,6 +13,7 @@
 // Both kernels are memory-latency work of a few hundred KB; they are written
 // for short, dependency-free loads (16-byte rows, no LDS staging of the
 // cache) and deterministic reductions (fixed orders, no float atomics).
+#include <algorithm>
 #include <cmath>
 
 #include "nibble_common.h"
@@ -25,11 +26,15 @@ namespace {
 
 constexpr int kHeadDim = 128;
 constexpr int kRopeHalf = kHeadDim / 2;
-constexpr int kChunk = 128;  // cached tokens per attention workgroup
+constexpr int kChunk = 128;     // tokens per chunk record the workspace has room for
+constexpr int kRound = 64;      // tokens an attention workgroup computes at a time
 constexpr int kGlueThreads = 256;
 constexpr int kRmsMaxCols = kRmsThreads * 8 * 8;
 constexpr int kAttnMaxSeq = 1 << 16;
-constexpr int kAttnMaxChunks = kAttnMaxSeq / kChunk;
+constexpr int kAttnMaxChunks = 64;     // chunks a launch uses at most
+constexpr int kAttnOneChunk = 384;     // tokens one workgroup takes alone
+constexpr int kAttnWorkgroups = 256;   // one round of the CUs
+constexpr int64_t kAttnRereadBytes = 80 << 20;  // cache bytes read by all parts together
 
 // y = fp16(x * r * w) with r = 1 / sqrt(mean(x^2) + eps), in fp32 (the
 // transformers LlamaRMSNorm computes the same in fp32 and rounds x * r to
@@ -69,9 +74,11 @@ struct AttnArgs {
   const float* rope_cos;   // [max_seq][64], or null: no rotary embedding
   const float* rope_sin;   // [max_seq][64]
   _Float16* out;           // [n_heads * 128]
-  float* partial;          // [n_kv][chunks][QPK][2 + 128] when chunks > 1
-  uint32_t* counters;      // [n_kv], zero on entry and on exit
-  int n_kv, max_seq, pos, chunks;
+  float* partial;          // [n_kv][chunks][qpk][2 + 128] when chunks > 1
+  uint32_t* counters;      // [n_kv * parts], zero on entry and on exit
+  int n_kv, max_seq, pos, qpk;
+  int chunks, chunk_tokens;  // chunk c: tokens [c chunk_tokens, ..); chunk_tokens a multiple of 64
+  int parts;               // workgroups sharing a kv head's query heads
 };
 
 // Element d of the rotary embedding of a 128-vector x at position pos, in the
@@ -84,42 +91,58 @@ __device__ __forceinline__ float rotate_half(_Float16 xd, _Float16 xp, float c, 
   return d < kRopeHalf ? v * c - static_cast<float>(xp) * s : v * c + static_cast<float>(xp) * s;
 }
 
-// Grouped-query attention of one decode token: QPK query heads share each
-// kv head.  Workgroup (h, c) takes kv head h, its QPK query heads and cached
-// tokens [128 c, min(128 c + 128, pos + 1)).  Token pos is the current one:
-// its k (rotated, rounded to fp16 as the cache holds it) and v come from qkv
-// and are written into the caches by the workgroup of the last chunk.
+// exp(x - m), 0 where x is -infinity (nothing seen) whatever m is.
+__device__ __forceinline__ float exp_below(float x, float m) {
+  return __expf(x - (m == -INFINITY ? 0.0f : m));
+}
+
+// Grouped-query attention of one decode token: qpk query heads share each kv
+// head.  Workgroup (h, c, part) takes HPW of kv head h's query heads and
+// cached tokens [c chunk_tokens, min(.. + chunk_tokens, pos + 1)).  Token pos
+// is the current one: its k (rotated, rounded to fp16 as the cache holds it)
+// and v come from qkv; the first part of the last chunk writes them into the
+// caches.
 //
-// 16 groups of 16 lanes each take every 16th token of the chunk; lane j of a
-// group holds dims 8j..8j+7 of the token's rows (one 16-byte load each).  All
-// of a lane's k and v rows are loaded at entry, before anything else: they
-// depend on nothing, so the chunk costs one memory round trip instead of one
-// per token.
-//   1. scores: per token, QPK dot products summed over the 16-lane group
-//      (one DPP row);
-//   2. softmax within the chunk: max, exp, sum per head (one wave a head);
-//   3. P V: each lane accumulates QPK x 8 outputs, then the 16 groups are
-//      summed in LDS in group order.
+// What bounds it: up to a few thousand tokens latency (launch, one round of
+// loads, the exchange between workgroups), beyond that the cache stream
+// (32768 tokens, 32 heads on 8: 4.4 TB/s).  Against one workgroup per kv head
+// and 128 tokens, softmax through LDS and a serial combine, us: 128 tokens
+// 6.0 -> 3.8, 1024 10.3 -> 7.5, 8192 29.5 -> 14.5, 32768 97.8 -> 30.7.
+// 16 groups of 16 lanes each take every 16th token; lane j of a group holds
+// dims 8j..8j+7 of a token's rows (one 16-byte load each).  A round is 64
+// tokens, 4 a group, the next round's rows in flight while one is computed:
+//   1. scores: HPW dot products a token, summed over the 16-lane group (DPP),
+//      so every lane has them;
+//   2. each group keeps its own running maximum, sum and P V (8 dims a lane)
+//      and rescales them when the maximum moves: no LDS and no barrier;
+//   3. at the end the 16 groups' maxima meet in LDS, each scales its sums to
+//      the common one, and the outputs are summed in group order.
 // With one chunk the output is written directly.  Otherwise each workgroup
 // publishes (max, sum, unnormalised P V) with device-coherent stores and the
-// last workgroup of the kv head (agent-scope counter) combines the chunks:
-// per head, the global max, the chunk weights exp(max_c - max) and the total
-// are formed in LDS (fixed order), then every output sums its chunks in chunk
-// order.  The first 8 to 32 chunks' partial outputs are loaded in the same
-// round as the maxima and sums.  Deterministic, one launch.
-template <int QPK>
+// last workgroup of (h, part) (agent-scope counter) combines the chunks: chunk
+// weights by one wave a head, then every output sums its chunks, all loads of
+// up to 16 chunks a thread issued before the weights are known.  Splitting the
+// query heads over workgroups (parts) spreads a short context over the CUs
+// without more partials, and shares out the combine; the cache rows are then
+// read by each part, from L2 (a kv head's workgroups sit on one XCD when n_kv
+// is a multiple of 8).  Deterministic, one launch.
+template <int HPW>
 __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs a) {
   constexpr int HD = kHeadDim;
-  constexpr int TPG = kChunk / 16;  // tokens per 16-lane group
-  constexpr float kScale = 0.08838834764831845f;  // 1 / sqrt(128)
-  __shared__ float qs[QPK][HD];
+  constexpr int TPG = kRound / 16;                 // tokens per 16-lane group and round
+  constexpr float kScale = 0.08838834764831845f;   // 1 / sqrt(128)
+  constexpr int SUBS = HPW >= 4 ? 1 : 4 / HPW;     // thread sets of the combine
+  constexpr int PAIRS = HPW * HD / 2;              // output pairs
+  constexpr int PER = (PAIRS + kGlueThreads - 1) / kGlueThreads;  // pairs per thread
+  constexpr int PRE = 16 / PER;                    // chunks a thread loads in one round
+  __shared__ float qs[HPW][HD];
   __shared__ __attribute__((aligned(16))) _Float16 knew[HD];
   __shared__ __attribute__((aligned(16))) _Float16 vnew[HD];
-  __shared__ float sc[QPK][kChunk];
-  __shared__ float red[16][QPK][HD];
-  __shared__ float mrow[QPK], lrow[QPK];
-  __shared__ float wchunk[kAttnMaxChunks][QPK];  // chunk max, then chunk weight
-  __shared__ float lchunk[kAttnMaxChunks][QPK];  // chunk sum
+  __shared__ __attribute__((aligned(16))) float red[16][HPW][HD];
+  __shared__ float mgrp[16][HPW], lgrp[16][HPW];
+  __shared__ float wchunk[kAttnMaxChunks][HPW];  // chunk max, then chunk weight
+  __shared__ float lchunk[kAttnMaxChunks][HPW];  // chunk sum
+  __shared__ float ltot[HPW];
   __shared__ int s_last;
 
   const int tid = threadIdx.x;
@@ -127,9 +150,11 @@ __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs
   const int wave = tid >> 6;
   const int h = blockIdx.x;
   const int c = blockIdx.y;
-  const int n_heads = a.n_kv * QPK;
-  const int t0 = c * kChunk;
-  const int t1 = min(t0 + kChunk, a.pos + 1);
+  const int part = blockIdx.z;
+  const int n_heads = a.n_kv * a.qpk;
+  const int head0 = h * a.qpk + part * HPW;        // this workgroup's first query head
+  const int t0 = c * a.chunk_tokens;
+  const int t1 = min(t0 + a.chunk_tokens, a.pos + 1);
   const size_t row0 = static_cast<size_t>(h) * a.max_seq;  // cache row of token 0
   const int g16 = tid >> 4;
   const int j = tid & 15;
@@ -141,14 +166,14 @@ __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs
   // Buffer loads without branches: a lane with nothing to load passes an
   // offset beyond the resource (it reads zero), and without rotary tables the
   // cos / sin resources are empty.
-  constexpr int QE = (QPK * HD + kGlueThreads - 1) / kGlueThreads;  // q elements per thread
+  constexpr int QE = (HPW * HD + kGlueThreads - 1) / kGlueThreads;  // q elements per thread
   const bool rope = a.rope_cos != nullptr;
   const uint32_t rope_bytes = rope ? static_cast<uint32_t>(a.max_seq) * kRopeHalf * 4u : 0u;
   const auto rq = make_rsrc(a.qkv, static_cast<uint32_t>(n_heads + 2 * a.n_kv) * HD * 2u);
   const auto rcos = make_rsrc(a.rope_cos, rope_bytes);
   const auto rsin = make_rsrc(a.rope_sin, rope_bytes);
   const uint32_t rope_row = static_cast<uint32_t>(a.pos) * kRopeHalf * 4u;
-  const bool writer = t1 == a.pos + 1 && tid < HD;  // writes the new token's k and v
+  const bool has_new = t1 == a.pos + 1 && tid < HD;  // holds the new token's k and v
   auto ld16 = [&](uint32_t off) {
     return __builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(rq, off, 0, 0));
   };
@@ -161,20 +186,20 @@ __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs
   for (int u = 0; u < QE; ++u) {
     const int e = tid + u * kGlueThreads;
     const int d = e % HD;
-    const uint32_t base = e < QPK * HD ? static_cast<uint32_t>(h * QPK * HD + e - d) * 2u
+    const uint32_t base = e < HPW * HD ? static_cast<uint32_t>(head0 * HD + e - d) * 2u
                                        : kOutOfRange;
-    const uint32_t rot = e < QPK * HD ? rope_row + static_cast<uint32_t>(d & (kRopeHalf - 1)) * 4u
+    const uint32_t rot = e < HPW * HD ? rope_row + static_cast<uint32_t>(d & (kRopeHalf - 1)) * 4u
                                       : kOutOfRange;
     qx[u] = ld16(base + static_cast<uint32_t>(d) * 2u);
     qp[u] = ld16(base + static_cast<uint32_t>(d ^ kRopeHalf) * 2u);
     qc[u] = ld32(rcos, rot);
     qn[u] = ld32(rsin, rot);
   }
-  const uint32_t kbase = writer ? static_cast<uint32_t>((n_heads + h) * HD) * 2u : kOutOfRange;
-  const uint32_t vbase = writer ? static_cast<uint32_t>((n_heads + a.n_kv + h) * HD) * 2u
+  const uint32_t kbase = has_new ? static_cast<uint32_t>((n_heads + h) * HD) * 2u : kOutOfRange;
+  const uint32_t vbase = has_new ? static_cast<uint32_t>((n_heads + a.n_kv + h) * HD) * 2u
+                                 : kOutOfRange;
+  const uint32_t krot = has_new ? rope_row + static_cast<uint32_t>(tid & (kRopeHalf - 1)) * 4u
                                 : kOutOfRange;
-  const uint32_t krot = writer ? rope_row + static_cast<uint32_t>(tid & (kRopeHalf - 1)) * 4u
-                               : kOutOfRange;
   const _Float16 kx0 = ld16(kbase + static_cast<uint32_t>(tid) * 2u);
   const _Float16 kxp = ld16(kbase + static_cast<uint32_t>(tid ^ kRopeHalf) * 2u);
   const _Float16 vx0 = ld16(vbase + static_cast<uint32_t>(tid) * 2u);
@@ -186,124 +211,142 @@ __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs
   const uint32_t head_bytes = static_cast<uint32_t>(a.max_seq) * HD * 2u;
   const auto rk = make_rsrc(a.k_cache + row0 * HD, head_bytes);
   const auto rv = make_rsrc(a.v_cache + row0 * HD, head_bytes);
-  h8_t kr[TPG], vr[TPG];
+  struct Rows {
+    h8_t k[TPG], v[TPG];
+  };
+  auto load = [&](Rows& r, int tb) {
 #pragma unroll
-  for (int u = 0; u < TPG; ++u) {
-    const int t = t0 + g16 + 16 * u;
-    const uint32_t off = t < t1 && t != a.pos ? static_cast<uint32_t>(t * HD + 8 * j) * 2u
-                                              : kOutOfRange;
-    kr[u] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0));
-    vr[u] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0));
-  }
+    for (int u = 0; u < TPG; ++u) {
+      const int t = tb + g16 + 16 * u;
+      const uint32_t off = t < t1 && t != a.pos ? static_cast<uint32_t>(t * HD + 8 * j) * 2u
+                                                : kOutOfRange;
+      r.k[u] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0));
+      r.v[u] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0));
+    }
+  };
+  Rows R0, R1;
+  load(R0, t0);
+  load(R1, t0 + kRound);
 
 #pragma unroll
   for (int u = 0; u < QE; ++u) {
     const int e = tid + u * kGlueThreads;
-    if (e < QPK * HD) {
+    if (e < HPW * HD) {
       const int hq = e / HD, d = e % HD;
       const float v = rope ? rotate_half(qx[u], qp[u], qc[u], qn[u], d) : static_cast<float>(qx[u]);
       qs[hq][d] = v * kScale;
     }
   }
-  if (writer) {
+  if (has_new) {
     const _Float16 kn = static_cast<_Float16>(
         rope ? rotate_half(kx0, kxp, kc, kn_s, tid) : static_cast<float>(kx0));
     knew[tid] = kn;
     vnew[tid] = vx0;
-    a.k_cache[(row0 + a.pos) * HD + tid] = kn;
-    a.v_cache[(row0 + a.pos) * HD + tid] = vx0;
+    if (part == 0) {
+      a.k_cache[(row0 + a.pos) * HD + tid] = kn;
+      a.v_cache[(row0 + a.pos) * HD + tid] = vx0;
+    }
   }
   __syncthreads();
 
-  float qr[QPK][8];
+  float qr[HPW][8], acc[HPW][8], m[HPW], l[HPW];
 #pragma unroll
-  for (int hq = 0; hq < QPK; ++hq)
+  for (int hq = 0; hq < HPW; ++hq) {
+    m[hq] = -INFINITY;
+    l[hq] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) qr[hq][i] = qs[hq][8 * j + i];
-#pragma unroll
-  for (int u = 0; u < TPG; ++u) {
-    const int t = t0 + g16 + 16 * u;
-    if (t == a.pos) {
-      kr[u] = *reinterpret_cast<const h8_t*>(&knew[8 * j]);
-      vr[u] = *reinterpret_cast<const h8_t*>(&vnew[8 * j]);
+    for (int i = 0; i < 8; ++i) {
+      qr[hq][i] = qs[hq][8 * j + i];
+      acc[hq][i] = 0.0f;
     }
-    // The whole 16-lane group (a DPP row) shares t, so all its lanes take
-    // part in the row sum.
-    if (t < t1) {
-      float s[QPK];
+  }
+  auto round = [&](Rows& r, int tb) {
+    float s[TPG][HPW];
 #pragma unroll
-      for (int hq = 0; hq < QPK; ++hq) {
-        s[hq] = 0.0f;
+    for (int u = 0; u < TPG; ++u) {
+      const int t = tb + g16 + 16 * u;
+      if (t == a.pos) {
+        r.k[u] = *reinterpret_cast<const h8_t*>(&knew[8 * j]);
+        r.v[u] = *reinterpret_cast<const h8_t*>(&vnew[8 * j]);
+      }
+#pragma unroll
+      for (int hq = 0; hq < HPW; ++hq) {
+        float d = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          s[hq] = __builtin_fmaf(qr[hq][i], static_cast<float>(kr[u][i]), s[hq]);
-        s[hq] = row16_sum(s[hq]);
-      }
-      if (j == 0) {
-#pragma unroll
-        for (int hq = 0; hq < QPK; ++hq) sc[hq][t - t0] = s[hq];
+          d = __builtin_fmaf(qr[hq][i], static_cast<float>(r.k[u][i]), d);
+        d = row16_sum(d);
+        s[u][hq] = t < t1 ? d : -INFINITY;
       }
     }
-  }
-  __syncthreads();
-
-  const int nt = t1 - t0;  // >= 1: the host sizes the grid so every chunk has a token
-  for (int hq = wave; hq < QPK; hq += kGlueThreads / 64) {
-    float m = -INFINITY;
-    for (int t = lane; t < nt; t += 64) m = fmaxf(m, sc[hq][t]);
-    m = wave_max(m);
-    float l = 0.0f;
-    for (int t = lane; t < nt; t += 64) {
-      const float p = __expf(sc[hq][t] - m);
-      sc[hq][t] = p;
-      l += p;
-    }
-    l = wave_sum(l);
-    if (lane == 0) {
-      mrow[hq] = m;
-      lrow[hq] = l;
-    }
-  }
-  __syncthreads();
-
-  float acc[QPK][8];
 #pragma unroll
-  for (int hq = 0; hq < QPK; ++hq)
+    for (int hq = 0; hq < HPW; ++hq) {
+      float top = m[hq];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[hq][i] = 0.0f;
+      for (int u = 0; u < TPG; ++u) top = fmaxf(top, s[u][hq]);
+      const float keep = exp_below(m[hq], top);
+      m[hq] = top;
+      l[hq] *= keep;
 #pragma unroll
-  for (int u = 0; u < TPG; ++u) {
-    const int t = t0 + g16 + 16 * u;
-    if (t < t1) {
+      for (int i = 0; i < 8; ++i) acc[hq][i] *= keep;
 #pragma unroll
-      for (int hq = 0; hq < QPK; ++hq) {
-        const float p = sc[hq][t - t0];
+      for (int u = 0; u < TPG; ++u) {
+        const float p = exp_below(s[u][hq], top);
+        l[hq] += p;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          acc[hq][i] = __builtin_fmaf(p, static_cast<float>(vr[u][i]), acc[hq][i]);
+          acc[hq][i] = __builtin_fmaf(p, static_cast<float>(r.v[u][i]), acc[hq][i]);
       }
     }
+  };
+  for (int tb = t0; tb < t1; tb += 2 * kRound) {
+    round(R0, tb);
+    load(R0, tb + 2 * kRound);
+    if (tb + kRound >= t1) break;
+    round(R1, tb + kRound);
+    load(R1, tb + 3 * kRound);
   }
+
+  // The groups' sums on the workgroup's common maximum.
+  if (j == 0) {
 #pragma unroll
-  for (int hq = 0; hq < QPK; ++hq)
+    for (int hq = 0; hq < HPW; ++hq) mgrp[g16][hq] = m[hq];
+  }
+  __syncthreads();
+  float top[HPW];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) red[g16][hq][8 * j + i] = acc[hq][i];
+  for (int hq = 0; hq < HPW; ++hq) {
+    top[hq] = mgrp[0][hq];
+#pragma unroll
+    for (int g = 1; g < 16; ++g) top[hq] = fmaxf(top[hq], mgrp[g][hq]);
+    const float w = exp_below(m[hq], top[hq]);
+    if (j == 0) lgrp[g16][hq] = l[hq] * w;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) red[g16][hq][8 * j + i] = acc[hq][i] * w;
+  }
   __syncthreads();
 
   const bool direct = a.chunks == 1;
-  for (int e = tid; e < QPK * HD; e += kGlueThreads) {
+  const size_t part_stride = static_cast<size_t>(a.qpk) * (HD + 2);  // floats per chunk
+  float* const P0 = a.partial + (static_cast<size_t>(h) * a.chunks * a.qpk + part * HPW) * (HD + 2);
+  for (int e = tid; e < HPW * HD; e += kGlueThreads) {
     const int hq = e / HD, d = e % HD;
-    float o = 0.0f;
+    float o = 0.0f, lsum = 0.0f;
 #pragma unroll
-    for (int g = 0; g < 16; ++g) o += red[g][hq][d];
+    for (int g = 0; g < 16; ++g) {
+      o += red[g][hq][d];
+      lsum += lgrp[g][hq];
+    }
     if (direct) {
-      a.out[static_cast<size_t>(h * QPK + hq) * HD + d] = static_cast<_Float16>(o / lrow[hq]);
+      a.out[static_cast<size_t>(head0 + hq) * HD + d] = static_cast<_Float16>(o / lsum);
     } else {
-      float* P = a.partial + ((static_cast<size_t>(h) * a.chunks + c) * QPK + hq) * (HD + 2);
+      float* P = P0 + c * part_stride + hq * (HD + 2);
       store_coherent(P + 2 + d, o);
       if (d == 0) {
-        store_coherent(P, mrow[hq]);
-        store_coherent(P + 1, lrow[hq]);
+        float t = mgrp[0][hq];
+        for (int g = 1; g < 16; ++g) t = fmaxf(t, mgrp[g][hq]);
+        store_coherent(P, t);
+        store_coherent(P + 1, lsum);
       }
     }
   }
@@ -313,87 +356,104 @@ __global__ __launch_bounds__(kGlueThreads) void attention_decode_kernel(AttnArgs
   // "HARDWARE ASSUMPTION" in nibble_decode.h.
   wait_vm_stores();
   __syncthreads();
+  uint32_t* counter = a.counters + h * a.parts + part;
   if (tid == 0) {
     const uint32_t prev =
-        __hip_atomic_fetch_add(a.counters + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = prev == static_cast<uint32_t>(a.chunks - 1);
   }
   __syncthreads();
   if (!s_last) return;
 
-  auto chunk_part = [&](int cc, int hq) {
-    return a.partial + ((static_cast<size_t>(h) * a.chunks + cc) * QPK + hq) * (HD + 2);
+  // Thread (sub, pair) sums output pairs `pair` (+ kGlueThreads) over the
+  // chunks sub, sub + SUBS, ...; the subs are added in order at the end.
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  const auto rp = make_rsrc(P0, static_cast<uint32_t>(a.chunks) * a.qpk * (HD + 2) * 4u);
+  auto ld_pair = [&](int cc, int hq, int d) {  // floats d, d + 1 of a chunk's record
+    const uint32_t off = cc < a.chunks
+                             ? (static_cast<uint32_t>(cc) * a.qpk + hq) * (HD + 2) * 4u + d * 4u
+                             : kOutOfRange;
+    return __builtin_bit_cast(f2_t, __builtin_amdgcn_raw_buffer_load_b64(rp, off, 0, 16));
   };
-  // One round of loads for up to PRE chunks: every chunk's (max, sum) into
-  // LDS, and this thread's partial outputs of the first PRE chunks into
-  // registers, all issued together.
-  constexpr int OUTS = (QPK * HD + kGlueThreads - 1) / kGlueThreads;  // outputs per thread
-  constexpr int PRE = 32 / OUTS;
-  float pv[OUTS][PRE];
+  const int sub = SUBS > 1 ? tid / PAIRS : 0;
+  const int pair = SUBS > 1 ? tid % PAIRS : tid;
+  f2_t pv[PER][PRE];
 #pragma unroll
-  for (int k = 0; k < OUTS; ++k) {
-    const int e = tid + k * kGlueThreads;
+  for (int k = 0; k < PER; ++k)
 #pragma unroll
-    for (int u = 0; u < PRE; ++u)
-      pv[k][u] = e < QPK * HD && u < a.chunks
-                     ? load_coherent(chunk_part(u, e / HD) + 2 + e % HD)
-                     : 0.0f;
-  }
-  for (int e = tid; e < a.chunks * QPK; e += kGlueThreads) {
-    const float* P = chunk_part(e / QPK, e % QPK);
-    const float mx = load_coherent(P);
-    const float sm = load_coherent(P + 1);
-    __builtin_amdgcn_sched_barrier(0);  // both loads in flight before either store waits
-    wchunk[e / QPK][e % QPK] = mx;
-    lchunk[e / QPK][e % QPK] = sm;
-  }
-  __syncthreads();
-  // Per head, over the chunks in order: the global max M, the chunk weights
-  // exp(max_c - M), and the total L = sum_c sum_c * weight_c.
-  if (tid < QPK) {
-    float M = -INFINITY;
-    for (int cc = 0; cc < a.chunks; ++cc) M = fmaxf(M, wchunk[cc][tid]);
-    mrow[tid] = M;
-  }
-  __syncthreads();
-  for (int e = tid; e < a.chunks * QPK; e += kGlueThreads) {
-    const int cc = e / QPK, hq = e % QPK;
-    wchunk[cc][hq] = __expf(wchunk[cc][hq] - mrow[hq]);
-  }
-  __syncthreads();
-  if (tid < QPK) {
-    float L = 0.0f;
-    for (int cc = 0; cc < a.chunks; ++cc) L += lchunk[cc][tid] * wchunk[cc][tid];
-    lrow[tid] = L;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < OUTS; ++k) {
-    const int e = tid + k * kGlueThreads;
-    if (e >= QPK * HD) continue;
-    const int hq = e / HD, d = e % HD;
-    float o = 0.0f;
-#pragma unroll
-    for (int u = 0; u < PRE; ++u)
-      if (u < a.chunks) o += pv[k][u] * wchunk[u][hq];
-    for (int c0 = PRE; c0 < a.chunks; c0 += 8) {  // beyond the prefetch: eight loads a round
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        v[u] = c0 + u < a.chunks ? load_coherent(chunk_part(c0 + u, hq) + 2 + d) : 0.0f;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (c0 + u < a.chunks) o += v[u] * wchunk[c0 + u][hq];
+    for (int u = 0; u < PRE; ++u) {
+      const int e = pair + k * kGlueThreads;
+      pv[k][u] = ld_pair(sub + u * SUBS, e / (HD / 2), 2 + 2 * (e % (HD / 2)));
     }
-    a.out[static_cast<size_t>(h * QPK + hq) * HD + d] = static_cast<_Float16>(o / lrow[hq]);
+  for (int e = tid; e < a.chunks * HPW; e += kGlueThreads) {
+    const f2_t ml = ld_pair(e / HPW, e % HPW, 0);
+    wchunk[e / HPW][e % HPW] = ml[0];
+    lchunk[e / HPW][e % HPW] = ml[1];
   }
-  if (tid == 0) __hip_atomic_store(a.counters + h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  for (int hq = wave; hq < HPW; hq += kGlueThreads / 64) {
+    float M = -INFINITY;
+    for (int cc = lane; cc < a.chunks; cc += 64) M = fmaxf(M, wchunk[cc][hq]);
+    M = wave_max(M);
+    float L = 0.0f;
+    for (int cc = lane; cc < a.chunks; cc += 64) {
+      const float w = exp_below(wchunk[cc][hq], M);
+      wchunk[cc][hq] = w;
+      L += lchunk[cc][hq] * w;
+    }
+    L = wave_sum(L);
+    if (lane == 0) ltot[hq] = L;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = pair + k * kGlueThreads;
+    const int hq = e / (HD / 2), d = 2 * (e % (HD / 2));
+    f2_t o = {0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < PRE; ++u) {
+      const int cc = sub + u * SUBS;
+      if (cc < a.chunks) {
+        const float w = wchunk[cc][hq];
+        o[0] += pv[k][u][0] * w;
+        o[1] += pv[k][u][1] * w;
+      }
+    }
+    for (int c0 = sub + PRE * SUBS; c0 < a.chunks; c0 += 8 * SUBS) {  // eight loads a round
+      f2_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = ld_pair(c0 + u * SUBS, hq, 2 + d);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (c0 + u * SUBS < a.chunks) {
+          const float w = wchunk[c0 + u * SUBS][hq];
+          o[0] += v[u][0] * w;
+          o[1] += v[u][1] * w;
+        }
+    }
+    if (SUBS > 1) {
+      red[sub][hq][d] = o[0];
+      red[sub][hq][d + 1] = o[1];
+    } else {
+      a.out[static_cast<size_t>(head0 + hq) * HD + d] = static_cast<_Float16>(o[0] / ltot[hq]);
+      a.out[static_cast<size_t>(head0 + hq) * HD + d + 1] = static_cast<_Float16>(o[1] / ltot[hq]);
+    }
+  }
+  if (SUBS > 1) {
+    __syncthreads();
+    for (int e = tid; e < HPW * HD; e += kGlueThreads) {
+      const int hq = e / HD, d = e % HD;
+      float o = red[0][hq][d];
+#pragma unroll
+      for (int s2 = 1; s2 < SUBS; ++s2) o += red[s2][hq][d];
+      a.out[static_cast<size_t>(head0 + hq) * HD + d] = static_cast<_Float16>(o / ltot[hq]);
+    }
+  }
+  if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-int attn_chunks(int64_t pos) { return static_cast<int>(ceil_div(pos + 1, kChunk)); }
-
 struct AttnPlan {
-  int qpk = 0, chunks = 0;
+  int qpk = 0, chunks = 0, chunk_tokens = 0, parts = 1;
   size_t counter_bytes = 0, workspace_bytes = 0;
 };
 
@@ -411,22 +471,46 @@ int plan_attention(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t max_
                "query heads per kv head must be 1, 2, 4 or 8, got %lld", (long long)qpk);
   NIBBLE_CHECK(pos >= 0 && pos < max_seq, "pos (%lld) must be in [0, max_seq = %lld)",
                (long long)pos, (long long)max_seq);
-  // The combine keeps every chunk's (max, sum) in LDS: at most 512 chunks.
   NIBBLE_CHECK(max_seq <= kAttnMaxSeq, "max_seq above %d", kAttnMaxSeq);
   p->qpk = static_cast<int>(qpk);
-  p->chunks = attn_chunks(pos);
-  if (p->chunks > 1) {
+  const int64_t tokens = pos + 1, room = ceil_div(tokens, kChunk);
+  if (room > 1) {
     p->counter_bytes = align_up(static_cast<size_t>(n_kv) * 4, 256);
-    p->workspace_bytes = p->counter_bytes + static_cast<size_t>(n_kv) * p->chunks * qpk *
+    p->workspace_bytes = p->counter_bytes + static_cast<size_t>(n_kv) * room * qpk *
                                                 (kHeadDim + 2) * sizeof(float);
   }
+  // Workgroups share a kv head's query heads between them, one head each, as
+  // long as reading the cache once per part stays cheap; the tokens are cut
+  // into as many chunks as make one round of the CUs (at least 128 tokens
+  // each: the workspace has room for no more).  Measured on MI355X, graph
+  // replay, 32 heads on 8, us: 1024 tokens 4 parts x 8 chunks 7.5 (1 part 9.5),
+  // 4096 tokens 4 x 8 10.6 (2 x 16 11.6, 1 x 32 13.4), 8192 tokens 2 x 16 14.5
+  // (4 x 8 15.7, 1 x 32 16.1), 32768 tokens 2 x 16 30.7 (4 x 16 45).  One chunk
+  // up to 384 tokens, which saves the exchange: 129 tokens 4.2 (2 chunks 6.2),
+  // 256 5.0 (6.3), 512 7.3 (4 chunks 6.7).
+  const int64_t cache_bytes = n_kv * tokens * kHeadDim * 4;
+  int64_t parts = qpk;
+  while (parts > 1 && ((parts > 2 && parts * cache_bytes > kAttnRereadBytes) ||
+                       n_kv * parts > 2 * kAttnWorkgroups ||
+                       (room > 1 && n_kv * parts > static_cast<int64_t>(p->counter_bytes / 4))))
+    parts /= 2;
+  const int64_t chunks =
+      tokens <= kAttnOneChunk
+          ? 1
+          : std::min<int64_t>({room, kAttnMaxChunks,
+                               std::max<int64_t>(1, kAttnWorkgroups / (n_kv * parts))});
+  const int64_t each = align_up(static_cast<size_t>(ceil_div(tokens, chunks)), kRound);
+  p->parts = static_cast<int>(parts);
+  p->chunk_tokens = static_cast<int>(each);
+  p->chunks = static_cast<int>(ceil_div(tokens, each));
   return NIBBLE_OK;
 }
 
-template <int QPK>
+template <int HPW>
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream) {
-  dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(a.chunks));
-  attention_decode_kernel<QPK><<<grid, kGlueThreads, 0, stream>>>(a);
+  dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(a.chunks),
+            static_cast<unsigned>(a.parts));
+  attention_decode_kernel<HPW><<<grid, kGlueThreads, 0, stream>>>(a);
   return hipGetLastError();
 }
 
@@ -534,10 +618,14 @@ extern "C" int nibble_attention_decode_f16(const void* QKV, int64_t n_heads, int
   a.max_seq = static_cast<int>(max_seq);
   a.pos = static_cast<int>(pos);
   a.chunks = p.chunks;
-  hipError_t e = p.qpk == 1   ? launch_attention<1>(a, stream)
-                 : p.qpk == 2 ? launch_attention<2>(a, stream)
-                 : p.qpk == 4 ? launch_attention<4>(a, stream)
-                              : launch_attention<8>(a, stream);
+  a.chunk_tokens = p.chunk_tokens;
+  a.parts = p.parts;
+  a.qpk = p.qpk;
+  const int heads_per_wg = p.qpk / p.parts;
+  hipError_t e = heads_per_wg == 1   ? launch_attention<1>(a, stream)
+                 : heads_per_wg == 2 ? launch_attention<2>(a, stream)
+                 : heads_per_wg == 4 ? launch_attention<4>(a, stream)
+                                     : launch_attention<8>(a, stream);
   NIBBLE_HIP(e);
   return ok();
 }

@@ -374,3 +374,25 @@ def test_glue_step_graph_replay():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
         step()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_heads,n_kv,pos", [
+    (32, 8, 63), (32, 8, 64), (32, 8, 127), (32, 8, 128), (32, 8, 383), (32, 8, 384), (32, 8, 1030),
+    (32, 8, 5200), (64, 8, 2600), (64, 8, 3000), (8, 8, 4095), (2, 2, 9000), (8, 1, 700), (16, 2, 12345),
+    (96, 96, 500), (192, 96, 130), (1024, 256, 400)])
+def test_attention_splits(n_heads, n_kv, pos):
+    """Every split of the work: one chunk up to 384 tokens, chunks cut at and
+    beside the 64-token rounds, one to eight query heads a workgroup, more
+    (kv head, part) pairs than counters.  Against the float32 reference to one
+    fp16 rounding of the output; repeats and replays give the same bits."""
+    max_seq = pos + 3
+    qkv, kc, vc = _attn_case(n_heads, n_kv, pos, max_seq, seed=pos + n_heads)
+    rope = glue.rope_tables(max_seq)
+    ref, k_row, v_row = ref_attention(qkv, kc, vc, pos, n_heads, n_kv, rope)
+    a = glue.attention_decode(qkv, kc, vc, pos, rope)
+    assert err_rms(a, ref) <= 1e-2
+    assert ulp_excess(a, ref) <= 1.0, ulp_excess(a, ref)
+    assert torch.equal(vc[:, pos], v_row)
+    for _ in range(20):
+        assert torch.equal(glue.attention_decode(qkv, kc, vc, pos, rope), a)
