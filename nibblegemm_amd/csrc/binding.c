@@ -267,6 +267,32 @@ static PyObject* py_dequant(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
+/* gemm_fuses(M, K, N, g) */
+static PyObject* py_gemm_fuses(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  (void)self;
+  if (!nargs_is(n, 4, "gemm_fuses")) return NULL;
+  long long M, K, N, g;
+  if (!take_i64(a[0], &M) || !take_i64(a[1], &K) || !take_i64(a[2], &N) || !take_i64(a[3], &g))
+    return NULL;
+  return PyBool_FromLong(nibble_gemm_fuses(M, K, N, g));
+}
+
+/* gemm_fused(X, xr, xc, Wq, S, K, N, g, sw, epilogue, bias, Y, ws, ws_bytes, stream) */
+static PyObject* py_gemm_fused(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  (void)self;
+  if (!nargs_is(n, 15, "gemm_fused")) return NULL;
+  void *X, *Wq, *S, *bias, *Y, *ws, *stream;
+  long long xr, xc, K, N, g, sw, ep, wsb;
+  if (!take_ptr(a[0], &X) || !take_i64(a[1], &xr) || !take_i64(a[2], &xc) ||
+      !take_ptr(a[3], &Wq) || !take_ptr(a[4], &S) || !take_i64(a[5], &K) ||
+      !take_i64(a[6], &N) || !take_i64(a[7], &g) || !take_i64(a[8], &sw) ||
+      !take_i64(a[9], &ep) || !take_ptr(a[10], &bias) || !take_ptr(a[11], &Y) ||
+      !take_ptr(a[12], &ws) || !take_i64(a[13], &wsb) || !take_ptr(a[14], &stream))
+    return NULL;
+  return PyLong_FromLong(nibble_gemm_w4a16_fused(X, xr, xc, Wq, S, K, N, g, sw, ep, bias, Y, ws,
+                                                 (size_t)(wsb < 0 ? 0 : wsb), stream));
+}
+
 /* quantize_rtn(W, K, N, dtype, g, Wq, S, stream) */
 static PyObject* py_quantize(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
@@ -415,6 +441,10 @@ static PyMethodDef kMethods[] = {
      "nibble_pack_strip_major"},
     {"gemv_strip_major", (PyCFunction)(void (*)(void))py_sm_gemv, METH_FASTCALL,
      "nibble_gemv_w4a16_strip_major"},
+    {"gemm_fuses", (PyCFunction)(void (*)(void))py_gemm_fuses, METH_FASTCALL,
+     "nibble_gemm_fuses"},
+    {"gemm_fused", (PyCFunction)(void (*)(void))py_gemm_fused, METH_FASTCALL,
+     "nibble_gemm_w4a16_fused"},
     {"quantize_rtn", (PyCFunction)(void (*)(void))py_quantize, METH_FASTCALL,
      "nibble_quantize_rtn"},
     {"gemm_strip_major", (PyCFunction)(void (*)(void))py_sm_gemm, METH_FASTCALL,

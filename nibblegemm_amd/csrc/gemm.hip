@@ -1154,3 +1154,46 @@ extern "C" int nibble_gemm_w4a16_strip_major(const void* X, int64_t x_rows, int6
   return gemm_run(X, x_rows, K, N, Wt, St, group_size, version, Y, workspace, workspace_bytes,
                   stream, strip_cols);
 }
+
+// nibble_gemm_w4a16 (version 6) with a fused output epilogue, on either
+// layout, for the shapes the direct kernel serves (no counterpart in the
+// reference, whose QuantLinear adds the bias as a separate fp16 op,
+// python/nibblegemm/ops.py:131-135).  The product's plan and sums are
+// nibble_gemm_w4a16's, so the outputs are the separate ops' bits.
+extern "C" int nibble_gemm_fuses(int64_t M, int64_t K, int64_t N, int64_t group_size) {
+  if ((group_size != 64 && group_size != 128) || M <= 8 || K <= 0 || N <= 0 || K % group_size != 0 ||
+      N % 2 != 0 || N >= kDirectMaxN || gemm_streams(M, K, N, group_size))
+    return 0;
+  return plan_tile(M, K, N, 6, nominal_bn_max(N), true).t.tm > 0 ? 1 : 0;
+}
+
+extern "C" int nibble_gemm_w4a16_fused(const void* X, int64_t x_rows, int64_t x_cols,
+                                       const void* Wq, const void* S, int64_t K, int64_t N,
+                                       int64_t group_size, int64_t strip_cols, int64_t epilogue,
+                                       const void* bias, void* Y, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
+  NIBBLE_CHECK(x_cols == K, "activation columns (%lld) disagree with K=%lld", (long long)x_cols,
+               (long long)K);
+  NIBBLE_CHECK(K > 0 && N > 0 && K % 8 == 0, "bad dimension (K and N must be positive)");
+  NIBBLE_CHECK(group_size == 64 || group_size == 128, "group_size must be 64 or 128");
+  NIBBLE_CHECK(K % group_size == 0, "K=%lld is not a multiple of group_size=%lld", (long long)K,
+               (long long)group_size);
+  NIBBLE_CHECK(strip_cols == 0 || strip_cols == 16 || strip_cols == 32 || strip_cols == 64,
+               "strip_cols must be 0 (packed), 16, 32 or 64, got %lld", (long long)strip_cols);
+  NIBBLE_CHECK(strip_cols == 0 || N % strip_cols == 0, "N=%lld is not a multiple of strip_cols=%lld",
+               (long long)N, (long long)strip_cols);
+  NIBBLE_CHECK(epilogue == kEpilogueBias || epilogue == kEpilogueSwiglu,
+               "epilogue must be 1 (bias) or 2 (swiglu), got %lld", (long long)epilogue);
+  NIBBLE_CHECK(epilogue != kEpilogueSwiglu || N % (2 * kSwigluBlock) == 0,
+               "swiglu needs N (gate|up interleaved in 16-column blocks) to be a multiple of 32");
+  NIBBLE_CHECK(epilogue != kEpilogueBias || x_rows == 0 || (bias != nullptr && aligned(bias, 2)),
+               "null or misaligned bias");
+  const int rc = validate_gemm(X, x_rows, x_cols, Wq, K / 8, N, S, K / group_size, N, group_size, 6,
+                               Y);
+  if (rc != NIBBLE_OK) return rc;
+  if (x_rows > 0 && !nibble_gemm_fuses(x_rows, K, N, group_size))
+    return fail(NIBBLE_ERR_UNSUPPORTED, "no fused epilogue for M=%lld K=%lld N=%lld",
+                (long long)x_rows, (long long)K, (long long)N);
+  return gemm_run(X, x_rows, K, N, Wq, S, group_size, 6, Y, workspace, workspace_bytes, stream,
+                  strip_cols, static_cast<int>(epilogue), bias);
+}

@@ -485,12 +485,52 @@ def _check_2d(X: torch.Tensor, qw: QuantizedWeight) -> None:
         raise ValueError(f"K mismatch: activations have {X.size(1)}, weights have {qw.K}")
 
 
+def _gemm_fusable(X: torch.Tensor, qw) -> bool:
+    """Whether a batch ``matmul`` would run on the direct GEMM kernel can have
+    its epilogue fused there (same plan, same bits): more than 8 rows that do
+    not stream, on either layout."""
+    W, S = qw.qweight, qw.scales
+    return (X.dim() == 2 and X.size(0) > DECODE_MAX_M and X.is_cuda and X.dtype == torch.float16
+            and X.is_contiguous() and X.data_ptr() % 16 == 0 and X.device == W.device == S.device
+            and W.dtype == torch.int32 and S.dtype == torch.float16
+            and W.is_contiguous() and S.is_contiguous()
+            and W.data_ptr() % 16 == 0 and S.data_ptr() % 16 == 0
+            and (isinstance(qw, StripMajorWeight)
+                 or (tuple(W.shape) == (qw.K // 8, qw.N)
+                     and tuple(S.shape) == (qw.K // max(qw.group_size, 1), qw.N)))
+            and _bind().gemm_fuses(X.size(0), qw.K, qw.N, qw.group_size))
+
+
+def _gemm_fused(X: torch.Tensor, qw, epilogue: int, bias: Optional[torch.Tensor],
+                n_out: int) -> torch.Tensor:
+    ext = _bind()
+    M, K = X.shape
+    dev = X.device
+    stream = _stream(dev)
+    Y = torch.empty((M, n_out), dtype=torch.float16, device=dev)
+    ws, ws_bytes = _gemm_workspace(ext, dev, stream, M, K, qw.N, qw.group_size, 6)
+    rc = ext.gemm_fused(X.data_ptr(), M, K, qw.qweight.data_ptr(), qw.scales.data_ptr(), K, qw.N,
+                        qw.group_size, qw.strip_cols if isinstance(qw, StripMajorWeight) else 0,
+                        epilogue, bias.data_ptr() if bias is not None else None, Y.data_ptr(),
+                        ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+    if rc:
+        _raise(rc, ext)
+    return Y
+
+
+def _tracked(t: torch.Tensor) -> bool:
+    """Whether autograd (reverse or forward mode) follows operations on ``t``:
+    those of a bias stay separate operations, which it records."""
+    return ((t.requires_grad and torch.is_grad_enabled())
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> torch.Tensor:
     """``matmul(X, qw) + bias`` -- the arithmetic of the reference's
     ``QuantLinear`` with a bias (ops.py:131-135): the fp16 product, then the
-    bias added in fp16.  An fp16 bias with M <= 128 runs as one launch (the
-    bias added in the kernel's epilogue, same bits); other cases run the two
-    ops."""
+    bias added in fp16.  An fp16 bias runs as one launch (the bias added in
+    the kernel's epilogue, same bits) wherever the kernel the product runs on
+    has one; other cases run the two ops."""
     _check_2d(X, qw)
     fp16_bias = (bias.dtype == torch.float16 and bias.dim() == 1 and bias.numel() == qw.N
                  and bias.device == X.device and bias.is_contiguous())
@@ -499,26 +539,34 @@ def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> tor
             return _strip_gemv(X, qw, 1, bias, qw.N)
     elif fp16_bias and _fusable(X, qw):
         return _fused(X, qw, 1, bias, qw.N)
+    if fp16_bias and not _tracked(bias) and _gemm_fusable(X, qw):
+        return _gemm_fused(X, qw, 1, bias, qw.N)
     return matmul(X, qw) + bias
 
 
 def matmul_swiglu(X: torch.Tensor, qw: QuantizedWeight) -> torch.Tensor:
     """``silu(X @ W_gate) * (X @ W_up)`` for ``qw = interleave_swiglu(gate,
     up)``, with the fp16 roundings of the unfused ops (the two products,
-    silu, then the product).  M <= 128 runs as one launch; so does a
+    silu, then the product), as one launch wherever the kernel the product
+    runs on has the epilogue: streamed batches of at most 128 rows, larger
+    ones on the direct GEMM kernel (either layout), and up to 8 rows a
     strip-major weight whose strips hold whole gate|up block pairs (at least
-    32 columns), while narrower strips compose the same arithmetic from the
-    plain product."""
+    32 columns).  Elsewhere the same arithmetic is composed from the plain
+    product."""
     _check_2d(X, qw)
     if qw.N % (2 * SWIGLU_BLOCK):
         raise ValueError(f"N={qw.N} is not an interleaved gate|up weight (multiple of 32)")
     if isinstance(qw, StripMajorWeight):
         if qw.strip_cols >= 2 * SWIGLU_BLOCK and X.size(0) <= DECODE_MAX_M:
             return _strip_gemv(X, qw, 2, None, qw.N // 2)
+        if _gemm_fusable(X, qw):
+            return _gemm_fused(X, qw, 2, None, qw.N // 2)
         gate, up = split_swiglu(_strip_gemm(X, qw))
         return torch.nn.functional.silu(gate) * up
     if _fusable(X, qw):
         return _fused(X, qw, 2, None, qw.N // 2)
+    if _gemm_fusable(X, qw):
+        return _gemm_fused(X, qw, 2, None, qw.N // 2)
     gate, up = split_swiglu(matmul(X, qw))
     return torch.nn.functional.silu(gate) * up
 

@@ -488,3 +488,41 @@ def test_workspace_plans_are_self_consistent(seed):
                 body = ws - cb
                 assert body % (4 * M * N) == 0, (kind, M, K, N, g, ws, cb)
                 assert 2 <= body // (4 * M * N) <= max_splits, (kind, M, K, N, g, ws, cb)
+
+
+def test_gemm_fused_validation():
+    """The fused GEMM entry refuses what it does not serve before any launch:
+    streamed batches, other epilogues, mismatched shapes, missing biases."""
+    ext = ng.extension()
+
+    def call(M=256, xc=512, K=512, N=256, g=128, sw=0, ep=1, bias=P, ptr=P):
+        return ext.gemm_fused(ptr, M, xc, ptr, ptr, K, N, g, sw, ep, bias, ptr, None, 0, None)
+
+    assert not ext.gemm_fuses(8, 512, 256, 128) and not ext.gemm_fuses(32, 4096, 4096, 128)
+    assert not ext.gemm_fuses(256, 512, 255, 128) and not ext.gemm_fuses(256, 500, 256, 128)
+    assert not ext.gemm_fuses(256, 512, 256, 32) and ext.gemm_fuses(256, 512, 256, 128)
+    assert not ext.gemm_fuses(129, 4096, 4096, 128)  # 64 x 128 tiles, which have no epilogue
+    for kwargs, needle in ((dict(xc=256), "disagree"), (dict(g=32), "group_size"), (dict(ep=0), "epilogue"),
+                           (dict(ep=2, N=272), "multiple of 32"), (dict(bias=None), "bias"),
+                           (dict(sw=48), "strip_cols"), (dict(sw=64, N=288), "multiple of strip_cols"),
+                           (dict(ptr=None), "null")):
+        assert call(**kwargs) == INVALID, kwargs
+        assert needle in ext.last_error(), (kwargs, ext.last_error())
+    assert call(M=32, xc=4096, K=4096, N=4096) not in (0, INVALID)
+    assert "no fused epilogue" in ext.last_error()
+    assert call(M=0) == 0
+
+
+def test_quantize_rtn_validation():
+    ext = ng.extension()
+
+    def call(K=256, N=64, dt=0, g=128, ptr=P):
+        return ext.quantize_rtn(ptr, K, N, dt, g, ptr, ptr, None)
+
+    for kwargs, needle in ((dict(K=200), "multiple of group_size"), (dict(g=12), "multiple of 8"),
+                           (dict(g=1024), "multiple of 8 up to"), (dict(dt=3), "dtype"),
+                           (dict(ptr=None), "null"), (dict(ptr=P + 1), "misaligned"),
+                           (dict(K=-128), "negative")):
+        assert call(**kwargs) == INVALID, kwargs
+        assert needle in ext.last_error(), (kwargs, ext.last_error())
+    assert call(N=0) == 0 and call(K=0) == 0

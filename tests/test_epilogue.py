@@ -139,3 +139,69 @@ def test_fused_plans_sharing_a_workspace():
         yg, yu = split_swiglu(ng.matmul(X2, qw))
         assert torch.equal(fused, torch.nn.functional.silu(yg) * yu)
         assert torch.equal(ng.matmul_bias(X1, w1, bias), ng.matmul(X1, w1) + bias)
+
+
+@pytest.mark.parametrize("M,K,N,g", [(129, 512, 256, 128), (200, 2048, 1088, 64), (1000, 576, 4102, 64),
+                                     (300, 8192, 1056, 128), (65, 4096, 14336, 128),
+                                     (512, 4096, 6016, 128), (700, 3072, 3008, 128)])
+def test_gemm_epilogues_are_the_separate_ops(M, K, N, g):
+    """Bias and SwiGLU on the direct GEMM kernel, with and without a K split
+    and two teams, on both layouts, into under-aligned outputs: the bits of the
+    product followed by the separate fp16 ops."""
+    ext = ng.extension()
+    assert ext.gemm_fuses(M, K, N, g)
+    _, _, _, Xd, qw = synthetic(M, K, N, g, seed=M + K)
+    weights = [qw]
+    if N % 64 == 0:
+        weights.append(ng.ops.to_strip_major(qw, 64))
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).half().to("cuda")
+    for w in weights:
+        y = ng.matmul(Xd, w)
+        want = y + bias
+        assert torch.equal(ng.matmul_bias(Xd, w, bias), want)
+        if N % 32 == 0:
+            gate, up = split_swiglu(y)
+            swiglu = torch.nn.functional.silu(gate) * up
+            assert torch.equal(ng.matmul_swiglu(Xd, w), swiglu)
+    # the C entry into outputs 2 bytes off: the same bits, nothing beside them
+    stream = torch.cuda.current_stream().cuda_stream
+    ws_bytes, _ = ext.gemm_workspace_bytes(M, K, N, g, 6, None)
+    ws = torch.zeros(max(ws_bytes, 256), dtype=torch.uint8, device="cuda")
+    for ep, out_n, ref in [(1, N, ng.matmul(Xd, qw) + bias)] + ([(2, N // 2, swiglu)] if N % 32 == 0 else []):
+        buf = torch.zeros(M * out_n + 8, dtype=torch.float16, device="cuda")
+        out = buf[1:1 + M * out_n]
+        rc = ext.gemm_fused(Xd.data_ptr(), M, K, qw.qweight.data_ptr(), qw.scales.data_ptr(), K, N, g,
+                            0, ep, bias.data_ptr(), out.data_ptr(), ws.data_ptr(), ws_bytes, stream)
+        assert rc == 0, ext.last_error()
+        assert torch.equal(out.view(M, out_n), ref)
+        assert buf[0] == 0 and buf[1 + M * out_n:].eq(0).all()
+
+
+def test_gemm_swiglu_of_extreme_products():
+    """Gates that overflow, underflow and are infinite or NaN, as the separate
+    ops handle them."""
+    M, K, N = 160, 256, 64
+    _, _, _, Xd, qw = synthetic(M, K, N, 128, seed=3)
+    X = Xd * 30
+    X[0] = float("inf")
+    X[1] = float("nan")
+    X[2] = 65504.0
+    X[3] = 0.0
+    assert ng.extension().gemm_fuses(M, K, N, 128)
+    gate, up = split_swiglu(ng.matmul(X, qw))
+    want = torch.nn.functional.silu(gate) * up
+    got = ng.matmul_swiglu(X, qw)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(nan=1.0), want.nan_to_num(nan=1.0))
+
+
+def test_bias_gradients_still_flow():
+    """A bias that autograd follows is added as a separate op."""
+    M, K, N = 160, 256, 64
+    _, _, _, Xd, qw = synthetic(M, K, N, 128, seed=3)
+    bias = torch.randn(N, device="cuda", dtype=torch.float16, requires_grad=True)
+    y = ng.matmul_bias(Xd, qw, bias)
+    y.float().sum().backward()
+    assert torch.allclose(bias.grad.float(), torch.full((N,), float(M), device="cuda"))
+    with torch.no_grad():
+        assert torch.equal(ng.matmul_bias(Xd, qw, bias), y.detach())
