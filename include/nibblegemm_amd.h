@@ -180,7 +180,7 @@ NIBBLE_API size_t nibble_gemm_counter_bytes(int64_t M, int64_t K, int64_t N, int
 NIBBLE_API int nibble_gemm_streams(int64_t M, int64_t K, int64_t N, int64_t group_size);
 
 /* nibble_gemm_w4a16 (version 6) with a fused output epilogue, for batches of
- * more than 8 rows that do not stream.  No counterpart in the reference, whose
+ * more than 8 rows, on either layout.  No counterpart in the reference, whose
  * QuantLinear adds the bias as a separate fp16 op
  * (python/nibblegemm/ops.py:131-135).  Epilogues 1 (bias) and 2 (SwiGLU of a
  * gate|up weight interleaved in 16-column blocks) as
@@ -188,8 +188,7 @@ NIBBLE_API int nibble_gemm_streams(int64_t M, int64_t K, int64_t N, int64_t grou
  * followed by the separate ops, to the bit.  `strip_cols` 0 reads packed
  * weights, else strip-major ones of that width.  Workspace as
  * nibble_gemm_workspace_bytes(M, K, N, group_size, 6).  nibble_gemm_fuses: 1
- * where this entry serves these sizes (weights 8-byte, scales 4-byte
- * aligned), else it returns NIBBLE_ERR_UNSUPPORTED.  ABI version 15. */
+ * where this entry serves these sizes (operands 16-byte aligned), else it returns NIBBLE_ERR_UNSUPPORTED.  ABI version 15. */
 NIBBLE_API int nibble_gemm_fuses(int64_t M, int64_t K, int64_t N, int64_t group_size);
 NIBBLE_API int nibble_gemm_w4a16_fused(const void* X, int64_t x_rows, int64_t x_cols,
                         const void* Wq, const void* S, int64_t K, int64_t N,

@@ -1023,13 +1023,12 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
     NIBBLE_HIP(fill_zero_f16(Y, M * N, stream));
     return ok();
   }
-  if (epilogue == kEpilogueNone && gemm_streams(M, K, N, group_size) &&
-      stream_supported(X, Wq, S, Y, M, K, N, group_size)) {
+  if (gemm_streams(M, K, N, group_size) && stream_supported(X, Wq, S, Y, M, K, N, group_size)) {
     StreamPlan p;
     rc = plan_stream(M, K, N, group_size, true, 0, 0, &p);
     if (rc != NIBBLE_OK) return rc;
     rc = launch_stream(X, Wq, S, Y, M, K, N, group_size, p, workspace, workspace_bytes, stream,
-                       "gemm (streaming) kernel launch", 0, nullptr, nullptr, 0.0f, strip_cols);
+                       "gemm (streaming) kernel launch", epilogue, bias, nullptr, 0.0f, strip_cols);
     return rc == NIBBLE_OK ? ok() : rc;
   }
   const auto* x = static_cast<const _Float16*>(X);
@@ -1156,14 +1155,15 @@ extern "C" int nibble_gemm_w4a16_strip_major(const void* X, int64_t x_rows, int6
 }
 
 // nibble_gemm_w4a16 (version 6) with a fused output epilogue, on either
-// layout, for the shapes the direct kernel serves (no counterpart in the
+// layout, for the shapes the streaming or direct kernels serve (no counterpart in the
 // reference, whose QuantLinear adds the bias as a separate fp16 op,
 // python/nibblegemm/ops.py:131-135).  The product's plan and sums are
 // nibble_gemm_w4a16's, so the outputs are the separate ops' bits.
 extern "C" int nibble_gemm_fuses(int64_t M, int64_t K, int64_t N, int64_t group_size) {
   if ((group_size != 64 && group_size != 128) || M <= 8 || K <= 0 || N <= 0 || K % group_size != 0 ||
-      N % 2 != 0 || N >= kDirectMaxN || gemm_streams(M, K, N, group_size))
+      N % 2 != 0 || N >= kDirectMaxN)
     return 0;
+  if (gemm_streams(M, K, N, group_size)) return 1;
   return plan_tile(M, K, N, 6, nominal_bn_max(N), true).t.tm > 0 ? 1 : 0;
 }
 

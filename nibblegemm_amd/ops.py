@@ -486,9 +486,8 @@ def _check_2d(X: torch.Tensor, qw: QuantizedWeight) -> None:
 
 
 def _gemm_fusable(X: torch.Tensor, qw) -> bool:
-    """Whether a batch ``matmul`` would run on the direct GEMM kernel can have
-    its epilogue fused there (same plan, same bits): more than 8 rows that do
-    not stream, on either layout."""
+    """Whether the kernel ``matmul`` runs this batch of more than 8 rows on
+    (either layout) takes the epilogue too (same plan, same bits)."""
     W, S = qw.qweight, qw.scales
     return (X.dim() == 2 and X.size(0) > DECODE_MAX_M and X.is_cuda and X.dtype == torch.float16
             and X.is_contiguous() and X.data_ptr() % 16 == 0 and X.device == W.device == S.device
@@ -548,11 +547,9 @@ def matmul_swiglu(X: torch.Tensor, qw: QuantizedWeight) -> torch.Tensor:
     """``silu(X @ W_gate) * (X @ W_up)`` for ``qw = interleave_swiglu(gate,
     up)``, with the fp16 roundings of the unfused ops (the two products,
     silu, then the product), as one launch wherever the kernel the product
-    runs on has the epilogue: streamed batches of at most 128 rows, larger
-    ones on the direct GEMM kernel (either layout), and up to 8 rows a
-    strip-major weight whose strips hold whole gate|up block pairs (at least
-    32 columns).  Elsewhere the same arithmetic is composed from the plain
-    product."""
+    runs on has the epilogue: nearly all do; up to 8 rows a strip-major weight
+    needs strips that hold whole gate|up block pairs (at least 32 columns).
+    Elsewhere the same arithmetic is composed from the plain product."""
     _check_2d(X, qw)
     if qw.N % (2 * SWIGLU_BLOCK):
         raise ValueError(f"N={qw.N} is not an interleaved gate|up weight (multiple of 32)")

@@ -492,13 +492,13 @@ def test_workspace_plans_are_self_consistent(seed):
 
 def test_gemm_fused_validation():
     """The fused GEMM entry refuses what it does not serve before any launch:
-    streamed batches, other epilogues, mismatched shapes, missing biases."""
+    other tiles and epilogues, mismatched shapes, missing biases."""
     ext = ng.extension()
 
     def call(M=256, xc=512, K=512, N=256, g=128, sw=0, ep=1, bias=P, ptr=P):
         return ext.gemm_fused(ptr, M, xc, ptr, ptr, K, N, g, sw, ep, bias, ptr, None, 0, None)
 
-    assert not ext.gemm_fuses(8, 512, 256, 128) and not ext.gemm_fuses(32, 4096, 4096, 128)
+    assert not ext.gemm_fuses(8, 512, 256, 128) and ext.gemm_fuses(32, 4096, 4096, 128)
     assert not ext.gemm_fuses(256, 512, 255, 128) and not ext.gemm_fuses(256, 500, 256, 128)
     assert not ext.gemm_fuses(256, 512, 256, 32) and ext.gemm_fuses(256, 512, 256, 128)
     assert not ext.gemm_fuses(129, 4096, 4096, 128)  # 64 x 128 tiles, which have no epilogue
@@ -508,7 +508,7 @@ def test_gemm_fused_validation():
                            (dict(ptr=None), "null")):
         assert call(**kwargs) == INVALID, kwargs
         assert needle in ext.last_error(), (kwargs, ext.last_error())
-    assert call(M=32, xc=4096, K=4096, N=4096) not in (0, INVALID)
+    assert call(M=129, xc=4096, K=4096, N=4096) not in (0, INVALID)
     assert "no fused epilogue" in ext.last_error()
     assert call(M=0) == 0
 
