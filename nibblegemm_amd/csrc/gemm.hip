@@ -4,10 +4,9 @@
 // checks :379-429).  The reference decodes B into shared memory and feeds
 // wmma / mma.sync; here the tile feeds v_mfma_f32_32x32x16_f16.
 //
-// Three kernels.  The direct kernel (gemm_direct.h) runs nearly everything;
-// gemm_pc64_kernel (further down) short batches over a middling K with few
-// tiles; gemm_tile_kernel, described here, the operands neither takes (odd N,
-// weights or scales not aligned for loads of two columns).
+// Two kernels.  The direct kernel (gemm_direct.h) runs nearly everything;
+// gemm_tile_kernel, described here, the operands it does not take (weights or
+// scales not aligned for loads of two columns, widths past its offsets).
 //
 // Tile: BM x BN x 32 per workgroup of 4 wave64s (2 x 2), each wave owning a
 // (BM/2) x (BN/2) block of 32 x 32 MFMA tiles.  Per 32-k step:
@@ -431,259 +430,18 @@ gemm_tile_kernel(TileArgs args) {
     __hip_atomic_store(args.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Epilogue of the producer/consumer kernel: the consumer waves hold the
-// results (wave block top-left (mw, nw), the tile kernel's register layout);
-// every wave passes the barriers of the K-split exchange.
-template <int TM, int TN, int THREADS, int BM, int BN>
-__device__ __forceinline__ void pc_epilogue(const f16_t (&acc)[TM][TN], const TileArgs& args,
-                                            bool producer, int mw, int nw, int& s_last) {
-  const int M = args.M, N = args.N;
-  const int lane = threadIdx.x & 63;
-  const int r32 = lane & 31;
-  const int rq = (lane >> 5) * 4;
-  _Float16* __restrict__ Y = args.Y;
-  if (args.splits == 1) {
-    if (producer) return;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int gn = nw + 32 * j + r32;
-        if (gn >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gm = mw + 32 * i + 8 * (r >> 2) + rq + (r & 3);
-          if (gm < M) Y[static_cast<size_t>(gm) * N + gn] = (_Float16)acc[i][j][r];
-        }
-      }
-    return;
-  }
-  float* part = args.partial + static_cast<size_t>(blockIdx.z) * M * N;
-  if (!producer) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int gn = nw + 32 * j + r32;
-        if (gn >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gm = mw + 32 * i + 8 * (r >> 2) + rq + (r & 3);
-          if (gm < M) store_coherent(part + static_cast<size_t>(gm) * N + gn, acc[i][j][r]);
-        }
-      }
-  }
-  // Last-arriver exchange; relies on gfx950 hardware ordering: see
-  // "HARDWARE ASSUMPTION" in nibble_decode.h.
-  wait_vm_stores();
-  __syncthreads();
-  const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-  if (threadIdx.x == 0) {
-    const uint32_t prev =
-        __hip_atomic_fetch_add(args.counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == static_cast<uint32_t>(args.splits - 1));
-  }
-  __syncthreads();
-  if (!s_last) return;
-  // Every wave (producers too) sums the tile: N % 4 == 0 for these kernels.
-  tile_sum_splits<THREADS, BM, BN>(args, static_cast<int>(blockIdx.y) * BM,
-                                   static_cast<int>(blockIdx.x) * BN);
-  if (threadIdx.x == 0)
-    __hip_atomic_store(args.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// LDS layout of the 64-k producer/consumer kernel: rows of 64 fp16 (eight
-// 16-byte units, 128 bytes, no padding), rows paired and XOR-swizzled by row
-// bits 0..5 so that the operand reads (16 consecutive rows, one unit),
-// A stores (2 rows x 8 units) and B stores (rows 4 apart, one unit) of every
-// 16-lane phase cover all 64 banks once (and every 8-lane phase all 32).
-__device__ __forceinline__ int lds_unit64(int r, int c) {
-  const int s0 = (r ^ (r >> 5)) & 1;
-  const int f = ((r ^ (r >> 3)) & 1) | (((r >> 1) ^ (r >> 4)) & 1) << 1 | ((r >> 2) & 1) << 2;
-  return 8 * ((r & ~1) | s0) + (c ^ f);
-}
-
-// Producer/consumer form of the tile kernel, with 64-k steps, 64 x 128 tiles:
-// four producer waves and four consumer waves (2 x 2, a 32 x 64 wave tile).
-// It serves short batches over a middling K whose few tiles are split over K
-// (plan_tile): there its narrower tiles make twice the workgroups of the
-// direct kernel's (gemm_direct.h), and the shorter chain of each wins --
-// 129 / 256 x 4096 x 4096 17.3 / 20.5 us against 18.5 / 21.8, 150 x 5120 x
-// 2048 15.0 against 16.5.
-//
-// The consumer waves only read operands from LDS and issue MFMAs (8 per wave
-// per step), while the producer waves run the global-load pipeline and the
-// decode, storing step t + 1 into the other LDS buffer while step t is
-// multiplied; the decode VALU work and the memory waits overlap the MFMAs.
-// Both roles pass the same barriers, ntiles + 1 of them, one per step.
-//
-// Producers: thread tid loads BM / 32 16-byte A chunks (rows tid / 8 + 32 it,
-// unit tid % 8) and one dwordx4 of B -- packed row tid / 32 of the step,
-// columns 4 (tid % 32) .. + 3 -- with its four scales.
-template <int GROUP>
-__global__ __launch_bounds__(8 * 64) void gemm_pc64_kernel(TileArgs args) {
-  constexpr int BM = 64, CWAVES = 4, PSTAGES = kStages;
-  constexpr int BN = 128;
-  constexpr int PBK = 64;
-  constexpr int THREADS = (CWAVES + 4) * 64;
-  constexpr int WROWS = CWAVES / 2;                  // consumer waves as WROWS x 2
-  constexpr int WM = BM / WROWS, WN = BN / 2;
-  constexpr int TM = WM / 32, TN = WN / 32;          // 32 x 32 MFMA tiles per wave
-  constexpr int A_IT = BM * (PBK / 8) / kGemmThreads;
-  __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * PBK];
-  __shared__ __attribute__((aligned(16))) _Float16 Bs[2][BN * PBK];
-  __shared__ int s_last;
-  const int M = args.M, K = args.K, N = args.N;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const bool producer = wave >= CWAVES;
-  const int tid = static_cast<int>(threadIdx.x) - (producer ? CWAVES * 64 : 0);
-  const int lane = tid & 63;
-  const int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
-  const int step0 = blockIdx.z * args.steps_per_split;
-  const int ntiles = min(args.steps_per_split, K / PBK - step0);
-  const int wm = (wave >> 1) % WROWS * WM;
-  const int wn = (wave & 1) * WN;
-  const int r32 = lane & 31;
-
-  f16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  if (producer) {
-    struct Stage {
-      h8_t a[A_IT];
-      u4_t b;
-      h4_t s;
-    };
-    const int prow = tid >> 5;
-    const int b_col = n0 + 4 * (tid & 31);
-    const uint32_t row_bytes = args.L.w_row;
-    const __amdgpu_buffer_rsrc_t rx =
-        make_rsrc(args.X, static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 2u);
-    const __amdgpu_buffer_rsrc_t rw =
-        make_rsrc(args.Wq, static_cast<uint32_t>(K / 8) * static_cast<uint32_t>(N) * 4u);
-    const __amdgpu_buffer_rsrc_t rsc =
-        make_rsrc(args.S, static_cast<uint32_t>(K / GROUP) * static_cast<uint32_t>(N) * 2u);
-    uint32_t voff_a[A_IT];
-    int a_st[A_IT];
-#pragma unroll
-    for (int it = 0; it < A_IT; ++it) {
-      const int row = (tid >> 3) + 32 * it;
-      const int gm = m0 + row;
-      voff_a[it] = gm < M ? (static_cast<uint32_t>(gm) * K + (tid & 7) * 8) * 2u : kOutOfRange;
-      a_st[it] = lds_unit64(row, tid & 7) * 8;
-    }
-    const bool b_ok = b_col < N;  // N % 4 == 0: the quad is wholly inside or outside
-    const uint32_t voff_b = b_ok ? prow * row_bytes + args.L.wcol(b_col) : kOutOfRange;
-    const uint32_t voff_s = b_ok ? args.L.scol(b_col) : kOutOfRange;
-    int b_st[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b_st[j] = lds_unit64(4 * (tid & 31) + j, prow) * 8;
-    auto load_step = [&](Stage& st, int step) {
-      const uint32_t k0 = static_cast<uint32_t>((step0 + min(step, ntiles - 1)) * PBK);
-#pragma unroll
-      for (int it = 0; it < A_IT; ++it)
-        st.a[it] = __builtin_bit_cast(
-            h8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, voff_a[it], k0 * 2u, 0));
-      st.b = __builtin_bit_cast(
-          u4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, voff_b, (k0 / 8) * row_bytes, 0));
-      st.s = __builtin_bit_cast(
-          h4_t, __builtin_amdgcn_raw_buffer_load_b64(
-                    rsc, voff_s, (k0 / GROUP) * args.L.s_row, 0));
-    };
-    auto store_step = [&](const Stage& st, int buf) {
-#pragma unroll
-      for (int it = 0; it < A_IT; ++it) *reinterpret_cast<h8_t*>(&As[buf][a_st[it]]) = st.a[it];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        h2_t w[4];
-        const h2_t s2 = {st.s[j], st.s[j]};
-        decode8_scaled(st.b[j], s2, w);
-        const h8_t v = {w[0][0], w[0][1], w[1][0], w[1][1], w[2][0], w[2][1], w[3][0], w[3][1]};
-        *reinterpret_cast<h8_t*>(&Bs[buf][b_st[j]]) = v;
-      }
-    };
-    // Ring of PSTAGES register stages: stage u holds step i while
-    // i % PSTAGES == u (each index is a compile-time constant).
-    Stage R[PSTAGES];
-#pragma unroll
-    for (int i = 0; i < PSTAGES; ++i) load_step(R[i], i);
-    auto piter = [&](auto u_const, int i) {
-      constexpr int u = decltype(u_const)::value;
-      store_step(R[u], i & 1);
-      load_step(R[u], i + PSTAGES);
-      __syncthreads();
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I3 = std::integral_constant<int, 3>;
-    int i = 0;
-    for (; i + PSTAGES <= ntiles; i += PSTAGES) {
-      piter(I0{}, i);
-      piter(I1{}, i + 1);
-      piter(I2{}, i + 2);
-      piter(I3{}, i + 3);
-    }
-    const int rem = ntiles - i;  // < PSTAGES
-    if (rem > 0) piter(I0{}, i);
-    if (rem > 1) piter(I1{}, i + 1);
-    if (rem > 2) piter(I2{}, i + 2);
-    __syncthreads();
-  } else {
-    int rda[TM][PBK / 16], rdb[TN][PBK / 16];
-#pragma unroll
-    for (int ks = 0; ks < PBK / 16; ++ks) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) rda[i][ks] = lds_unit64(wm + 32 * i + r32, 2 * ks + (lane >> 5)) * 8;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) rdb[j][ks] = lds_unit64(wn + 32 * j + r32, 2 * ks + (lane >> 5)) * 8;
-    }
-    __syncthreads();
-    for (int t = 0; t < ntiles; ++t) {
-      const int buf = t & 1;
-#pragma unroll
-      for (int ks = 0; ks < PBK / 16; ++ks) {
-        h8_t a[TM], b[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const h8_t*>(&As[buf][rda[i][ks]]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const h8_t*>(&Bs[buf][rdb[j][ks]]);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(a[i], b[j], acc[i][j]);
-      }
-      __syncthreads();
-    }
-  }
-  pc_epilogue<TM, TN, THREADS, BM, BN>(acc, args, producer, m0 + wm, n0 + wn, s_last);
-}
-
-hipError_t launch_pc64(const TileArgs& a, int64_t G, hipStream_t stream) {
-  dim3 grid(static_cast<unsigned>(ceil_div(a.N, 128)), static_cast<unsigned>(ceil_div(a.M, 64)),
-            static_cast<unsigned>(a.splits));
-  if (G == 128)
-    gemm_pc64_kernel<128><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
-  else
-    gemm_pc64_kernel<64><<<grid, 2 * kGemmThreads, 0, stream>>>(a);
-  return hipGetLastError();
-}
-
-template <int TM, int KW>
-hipError_t launch_direct_cfg(const DirectArgs& a, int64_t G, hipStream_t stream) {
-  // Up to 4 row tiles a wave leaves registers for two waves per SIMD.
-  constexpr int kOcc = TM <= 4 ? 2 : 1;
+template <int TM, int KW, int WN>
+hipError_t launch_direct_cfg(DirectArgs a, int64_t G, hipStream_t stream) {
+  // Up to 3 row tiles (4 with four waves side by side) a wave leaves registers
+  // for two waves per SIMD.
+  constexpr int kOcc = TM <= 2 || (TM <= 4 && KW * WN >= 4 && WN == 4) ? 2 : 1;
+  a.tiles_m = static_cast<int>(ceil_div(a.M, 32 * TM));
+  a.tiles_n = static_cast<int>(ceil_div(a.N, 64 * WN));
   const unsigned grid = static_cast<unsigned>(a.tiles_m) * a.tiles_n * a.splits;
   if (G == 128)
-    gemm_direct_kernel<TM, KW, 128, kOcc><<<grid, KW * kDirectWaves * 64, 0, stream>>>(a);
+    gemm_direct_kernel<TM, KW, WN, 128, kOcc><<<grid, KW * WN * 64, 0, stream>>>(a);
   else
-    gemm_direct_kernel<TM, KW, 64, kOcc><<<grid, KW * kDirectWaves * 64, 0, stream>>>(a);
+    gemm_direct_kernel<TM, KW, WN, 64, kOcc><<<grid, KW * WN * 64, 0, stream>>>(a);
   return hipGetLastError();
 }
 
@@ -699,12 +457,10 @@ hipError_t launch_tile(const TileArgs& a, int64_t G, hipStream_t stream) {
 }
 
 // Which kernel a call runs, and its tile: the direct kernel's (tm > 0: 32 tm
-// rows by 256 columns, kw teams), the producer/consumer kernel's 64 x 128, or
-// the tile kernel's bm x bn.
+// rows by 64 wn columns, kw teams), else the tile kernel's bm x bn.
 struct TileChoice {
   int bm, bn;
-  bool pc = false;
-  int tm = 0, kw = 1;
+  int tm = 0, kw = 1, wn = 4;
 };
 
 // The device the plans are made for: MI355X, 256 CUs.  Planning with a fixed
@@ -716,7 +472,7 @@ constexpr int kPlanCUs = 256;
 int nominal_bn_max(int64_t N) { return N % 4 == 0 ? 256 : N % 2 == 0 ? 128 : 64; }
 
 // k per pipeline step of the kernel a choice runs.
-int step_k(TileChoice t) { return t.pc || t.tm > 0 ? 64 : BK; }
+int step_k(TileChoice t) { return t.tm > 0 ? kDirectStep : BK; }
 
 // Widest B vector (BN / 64 packed words per thread) the operands allow.
 int max_bn(int64_t N, const void* w, const void* s) {
@@ -725,8 +481,8 @@ int max_bn(int64_t N, const void* w, const void* s) {
   return 64;
 }
 
-// Tile choice of the tile kernel (the shapes the producer/consumer kernel
-// does not take), measured on MI355X over M = 64..2048 at 4096 x 14336 and
+// Tile choice of the tile kernel (the shapes the direct kernel does not
+// take), measured on MI355X over M = 64..2048 at 4096 x 14336 and
 // 14336 x 4096: 128 x 128 (2 waves per SIMD, so one workgroup's barrier
 // wait overlaps another's MFMAs) is fastest whenever its grid gives every CU
 // a workgroup; otherwise 64 x 128, whose doubled grid wins (e.g. 126 us vs
@@ -756,18 +512,18 @@ TilePlan plan_split_room(int64_t M, int64_t K, int64_t N, int64_t version, int b
   TilePlan p;
   int64_t tiles = 0;
   int splits = 1;
+  int unit = 64;  // k the splits are cut in
   if (M <= kStreamMaxM && K % 64 == 0 && bn_max >= 256) {
     // Small batches that do not stream (gemm_streams): the largest of 1, 2, 4,
     // 8 ways keeping the grid of 64-row tiles within 320 workgroups.  Both
     // versions take this plan (so they agree to the bit).
-    p.t = TileChoice{64, 128, true};
+    p.t = TileChoice{64, 128};
     tiles = ceil_div(M, 64) * ceil_div(N, 128);
     while (splits < 8 && tiles * splits * 2 <= 320 && K / 64 >= 2 * splits) splits *= 2;
   } else if (K % 64 == 0 && bn_max >= 256) {
     const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
-    const int bm = version == 7 || K >= 8192 || t128 >= 192 ? 128 : 64;
-    p.t = TileChoice{bm, 128, bm == 64};
-    tiles = ceil_div(M, bm) * ceil_div(N, 128);
+    p.t = TileChoice{version == 7 || K >= 8192 || t128 >= 192 ? 128 : 64, 128};
+    tiles = ceil_div(M, p.t.bm) * ceil_div(N, 128);
     if (K >= 8192) {
       if (tiles <= 64)
         splits = 4;
@@ -775,18 +531,19 @@ TilePlan plan_split_room(int64_t M, int64_t K, int64_t N, int64_t version, int b
         splits = 2;
       else if (tiles > kPlanCUs && tiles < 2 * kPlanCUs)
         splits = 2;
-    } else if (bm == 64 && K >= 4096 && tiles <= 160) {
+    } else if (p.t.bm == 64 && K >= 4096 && tiles <= 160) {
       splits = 4;
     }
   } else {
+    unit = BK;
     p.t = version == 7 ? TileChoice{128, std::min(128, bn_max)} : choose_tile(M, N, bn_max);
     tiles = ceil_div(M, p.t.bm) * ceil_div(N, p.t.bn);
     if (K >= 8192 && tiles < 2 * kPlanCUs)
       splits = static_cast<int>(std::min<int64_t>(ceil_div(2 * kPlanCUs, tiles), 4));
   }
-  const int steps = static_cast<int>(K / step_k(p.t));
-  p.steps_per_split = static_cast<int>(ceil_div(steps, splits));
-  p.splits = static_cast<int>(ceil_div(steps, p.steps_per_split));
+  const int64_t steps = K / unit, per = ceil_div(steps, splits);
+  p.steps_per_split = static_cast<int>(per * (unit / BK));
+  p.splits = static_cast<int>(ceil_div(steps, per));
   if (p.splits > 1) {
     p.counter_bytes = align_up(static_cast<size_t>(tiles) * 4, 256);
     p.workspace_bytes = p.counter_bytes + static_cast<size_t>(p.splits) * M * N * 4;
@@ -804,49 +561,49 @@ bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
 
 // The direct kernel's tile, teams and splits for a shape, within the splits
 // and counters of `room`.  A model of its time, fitted to MI355X measurements
-// of every tile at some 30 shapes (M = 33..4096), us: 4.5 to start and drain;
-// per 64-k step and round of the CUs the tile's own time when few workgroups
-// run, kStep; 0.36 of the time the whole product takes at the power-limited
-// 1.25 PFLOP/s; and for a K split 3 plus its partials at 2.5 TB/s.  Tiles of
-// up to 4 row tiles share a CU two at a time, so their last round is half as
-// dear.  It names the fastest tile or one within ~5% at nearly all of them:
-// e.g. 512 x 4096 x 14336 tm = 4 55 us (3: 69, 8: 75), 1000 x 5504 x 4102
-// tm = 3 50 (4: 55), 256 x 4096 x 14336 tm = 2 33 (4: 40, 8: 72), 3000 x
-// 3072 x 3008 tm = 5 54 (3: 57, 4: 66), 129 x 14336 x 4096 tm = 2, 4 splits
-// 32 (unsplit 77), 4096 x 4096 x 4096 tm = 8 108 (4: 111).
-// Up to 96 rows a tile, two teams halve a long K within the workgroup; K <
-// 2048 is too short for that to pay.
+// of every tile and split at some 40 shapes (M = 33..4096), us: 4.5 to start
+// and drain; per 64-k step and round of the CUs the tile's own time, `step`;
+// 0.36 of the time the whole product takes at the power-limited 1.25 PFLOP/s;
+// and for a K split 2 plus its partials at 2 TB/s.  `tail` is how much of a
+// part-filled last round is paid for (less where two workgroups share a CU).
+// It names the fastest plan at most of them and one within ~7% at the rest:
+// 96 x 8192 x 8192 (M x K x N) tm = 2, 4 teams, 2 columns waves, 2 splits
+// 23.2 us (tm = 1, 2 teams, 4 column waves 26.9), 128 x 4096 x 14336 the same
+// unsplit 19.0 (25.2), 256 x 4096 x 4096 tm = 1, 4 teams 14.9 (2 teams, 2
+// splits 21.8), 512 x 4096 x 14336 tm = 4 52.5 (2: 61, 8: 75), 1000 x 5504 x
+// 4102 tm = 3, 2 teams 48 (4: 54), 3000 x 3072 x 3008 tm = 5 54 (3: 57, 4:
+// 66), 4096 x 4096 x 4096 tm = 8 108 (4: 111).
+// Teams split K, so a K below 1024 keeps one.
 TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, int* splits) {
   struct Cfg {
-    int tm;
-    double step, step2;  // one team, two teams
+    int tm, kw, wn;
+    double step, tail;
   };
-  static constexpr Cfg kCfgs[] = {{1, 0.36, 0.28}, {2, 0.40, 0.36}, {3, 0.45, 0.40},
-                                  {4, 0.53, 0.0},  {5, 0.68, 0.0},  {6, 0.80, 0.0},
-                                  {8, 1.03, 0.0}};
-  const int64_t tiles_n = ceil_div(N, kDirectBN), steps = K / kDirectStep;
+  static constexpr Cfg kCfgs[] = {
+      {1, 4, 2, 0.127, 0.75}, {2, 4, 2, 0.155, 1.0}, {3, 2, 2, 0.215, 1.0}, {4, 2, 2, 0.275, 1.0},
+      {2, 2, 4, 0.31, 1.0},   {3, 2, 4, 0.37, 1.0},  {1, 1, 4, 0.36, 0.5},  {2, 1, 4, 0.40, 0.5},
+      {3, 1, 4, 0.45, 0.5},   {4, 1, 4, 0.52, 0.5},  {5, 1, 4, 0.68, 1.0},  {6, 1, 4, 0.80, 1.0},
+      {8, 1, 4, 1.03, 1.0}};
+  const int64_t steps = K / kDirectStep;
   const int64_t max_counters = static_cast<int64_t>(room.counter_bytes / 4);
   const double power = 0.36 * 2.0 * static_cast<double>(M) * K * N / 1.25e9;
-  TileChoice best{0, kDirectBN};
+  TileChoice best{0, 0};
   double best_us = 1e30;
   for (const Cfg& c : kCfgs) {
-    const bool teams = c.step2 > 0 && K >= 2048;
-    const double step = teams ? c.step2 : c.step;
-    const int64_t tiles = ceil_div(M, 32 * c.tm) * tiles_n;
+    if (c.kw > 1 ? K < 1024 : c.tm <= 3 && K >= 1024) continue;
+    const int64_t tiles = ceil_div(M, 32 * c.tm) * ceil_div(N, 64 * c.wn);
     for (int s = 1; s <= (c.tm <= kDirectMaxSplitTM ? room.splits : 1); ++s) {
       if (s > 1 && tiles > max_counters) break;
       const int64_t per = ceil_div(steps, s);
-      if (ceil_div(steps, per) != s) continue;  // not a split count that divides evenly enough
+      if (ceil_div(steps, per) != s) continue;  // those steps make fewer splits
       const double fill = static_cast<double>(tiles * s) / kPlanCUs;
       const double rounds = static_cast<double>(ceil_div(tiles * s, kPlanCUs));
-      const double eff = c.tm <= 4 && fill > 1 ? 0.5 * (rounds + fill) : rounds;
-      double us = 4.5 + eff * static_cast<double>(per) * step + power;
-      if (s > 1) us += 3.0 + static_cast<double>(s) * M * N * 4 / 2.5e6;
+      const double eff = fill > 1 ? c.tail * rounds + (1.0 - c.tail) * fill : rounds;
+      double us = 4.5 + eff * static_cast<double>(per) * c.step + power;
+      if (s > 1) us += 2.0 + static_cast<double>(s) * M * N * 4 / 2.0e6;
       if (us < best_us) {
         best_us = us;
-        best.bm = 32 * c.tm;
-        best.tm = c.tm;
-        best.kw = teams ? 2 : 1;
+        best = TileChoice{32 * c.tm, 64 * c.wn, c.tm, c.kw, c.wn};
         *splits = s;
       }
     }
@@ -859,9 +616,7 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
 // to the bit.
 TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max, bool direct) {
   TilePlan p = plan_split_room(M, K, N, version, bn_max);
-  // The 64 x 128 tiles keep the mid-K shapes they are split 4 ways for.
-  const bool mid_k = M > kStreamMaxM && p.t.pc && p.splits > 1;
-  if (direct && !mid_k) {
+  if (direct) {
     int splits = 1;
     p.t = choose_direct(M, K, N, p, &splits);
     p.splits = splits;
@@ -870,26 +625,26 @@ TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max,
   return p;
 }
 
-hipError_t launch_direct(TileChoice t, DirectArgs a, int64_t G, hipStream_t stream) {
-  a.tiles_m = static_cast<int>(ceil_div(a.M, 32 * t.tm));
-  a.tiles_n = static_cast<int>(ceil_div(a.N, kDirectBN));
-  switch (t.tm * 2 + t.kw - 1) {
-    case 2: return launch_direct_cfg<1, 1>(a, G, stream);
-    case 3: return launch_direct_cfg<1, 2>(a, G, stream);
-    case 4: return launch_direct_cfg<2, 1>(a, G, stream);
-    case 5: return launch_direct_cfg<2, 2>(a, G, stream);
-    case 6: return launch_direct_cfg<3, 1>(a, G, stream);
-    case 7: return launch_direct_cfg<3, 2>(a, G, stream);
-    case 8: return launch_direct_cfg<4, 1>(a, G, stream);
-    case 10: return launch_direct_cfg<5, 1>(a, G, stream);
-    case 12: return launch_direct_cfg<6, 1>(a, G, stream);
-    case 16: return launch_direct_cfg<8, 1>(a, G, stream);
+hipError_t launch_direct(TileChoice t, const DirectArgs& a, int64_t G, hipStream_t stream) {
+  switch (t.tm * 100 + t.kw * 10 + t.wn) {
+    case 142: return launch_direct_cfg<1, 4, 2>(a, G, stream);
+    case 242: return launch_direct_cfg<2, 4, 2>(a, G, stream);
+    case 322: return launch_direct_cfg<3, 2, 2>(a, G, stream);
+    case 422: return launch_direct_cfg<4, 2, 2>(a, G, stream);
+    case 224: return launch_direct_cfg<2, 2, 4>(a, G, stream);
+    case 324: return launch_direct_cfg<3, 2, 4>(a, G, stream);
+    case 114: return launch_direct_cfg<1, 1, 4>(a, G, stream);
+    case 214: return launch_direct_cfg<2, 1, 4>(a, G, stream);
+    case 314: return launch_direct_cfg<3, 1, 4>(a, G, stream);
+    case 414: return launch_direct_cfg<4, 1, 4>(a, G, stream);
+    case 514: return launch_direct_cfg<5, 1, 4>(a, G, stream);
+    case 614: return launch_direct_cfg<6, 1, 4>(a, G, stream);
+    case 814: return launch_direct_cfg<8, 1, 4>(a, G, stream);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_choice(TileChoice t, const TileArgs& a, int64_t G, hipStream_t stream) {
-  if (t.pc) return launch_pc64(a, G, stream);
   if (t.bm == 128 && t.bn == 128) return launch_tile<128, 128>(a, G, stream);
   if (t.bm == 64 && t.bn == 128) return launch_tile<64, 128>(a, G, stream);
   if (t.bm == 128 && t.bn == 64) return launch_tile<128, 64>(a, G, stream);
@@ -942,14 +697,12 @@ namespace {
 // 16-row MFMA tiles), where a 64/128-row tile would leave most of the device
 // idle.  Measured on MI355X at K=4096, N=14336: M=16 takes 82 us through the
 // tile kernel and 11 us streaming.  Above 32 rows streaming takes one pass
-// per 32 rows; once those passes would move 48 MiB or more, 64-row tiles of
-// the producer/consumer kernel with a K split win (plan_tile).  Measured,
-// graph replay, streaming against tiles: 4096 x 14336 M = 48 / 64 / 128
-// 21.0 / 23.7 / 41.9 us against 19.6 / 20.1 / 26.5; 14336 x 4096 M = 33 /
-// 64 / 128 23.1 / 31.6 / 56.6 against 20.6 / 21.9 / 29.3; 8192 x 8192
-// M = 33 25.0 against 19.6; 4096 x 6144 M = 128 22.0 against 19.0.  Below
-// that streaming stays ahead: 4096 x 4096 M = 33..128 12.4-12.6 us against
-// 12.9-14.4, 4096 x 6144 M = 64 12.7 against 14.0.
+// per 32 rows; once those passes would move 48 MiB or more, the direct
+// kernel's tiles win (plan_tile).  Measured, graph replay, streaming against
+// tiles: 4096 x 14336 M = 65 / 128 25 / 41.9 us against 17.2 / 19.0; 14336 x
+// 4096 M = 128 56.6 against 23.6; 8192 x 8192 M = 96 43 against 23.2.  Below
+// that streaming stays ahead or level: 4096 x 4096 M = 33..128 10.6-12.6 us
+// against 12.9-14.0, 4096 x 6144 M = 64 12.7 against 14.0.
 bool gemm_streams(int64_t M, int64_t K, int64_t N, int64_t G) {
   if (!(M >= 1 && M <= kStreamMaxM && K > 0 && N > 0 && N % 4 == 0 && K % G == 0)) return false;
   const int64_t pass_bytes = K * N / 2;
@@ -1052,9 +805,9 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
   const TilePlan nominal = bn_max == nominal_bn_max(N) && direct == nominal_direct
                                ? p
                                : plan_tile(M, K, N, version, nominal_bn_max(N), nominal_direct);
-  if (M > rows_max || gemm_streams(M, K, N, group_size) || p.t.pc != nominal.t.pc ||
-      p.t.tm != nominal.t.tm || p.t.kw != nominal.t.kw || p.t.bm != nominal.t.bm ||
-      p.t.bn != nominal.t.bn || p.splits != nominal.splits)
+  if (M > rows_max || gemm_streams(M, K, N, group_size) || p.t.tm != nominal.t.tm ||
+      p.t.kw != nominal.t.kw || p.t.bm != nominal.t.bm || p.t.bn != nominal.t.bn ||
+      p.splits != nominal.splits)
     p.splits = 1;
   if (p.splits > 1) {
     if (workspace == nullptr || workspace_bytes < p.workspace_bytes)

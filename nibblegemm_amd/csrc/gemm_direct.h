@@ -49,11 +49,9 @@ __device__ __forceinline__ f16_t mfma32(h8_t a, h8_t b, f16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-constexpr int kDirectWaves = 4;            // waves side by side along N (one K team)
-constexpr int kDirectBN = 64 * kDirectWaves;
 constexpr int kDirectStep = 64;            // k per step
 constexpr int kDirectRing = 4;             // activation buffers (and word sets) per team
-constexpr int kDirectMaxSplitTM = 4;       // larger tiles are never split over K
+constexpr int kDirectMaxSplitTM = 3;       // larger tiles are never split over K
 constexpr int kPolicyCoherent = 16;        // sc1: the cache policy of an agent-scope access
 constexpr int kDirectGroupM = 8;           // row tiles per block of the tile order
 
@@ -195,12 +193,12 @@ struct PartialVec<2> {
   }
 };
 
-template <int THREADS, int BM, int VEC>
+template <int THREADS, int BM, int BN, int VEC>
 __device__ __forceinline__ void direct_sum_splits(const DirectArgs& args, int m0, int n0) {
   using P = PartialVec<VEC>;
   using vec = typename P::type;
   constexpr int kBatch = 4, kPair = 2;
-  constexpr int CHUNKS = BM * kDirectBN / VEC;
+  constexpr int CHUNKS = BM * BN / VEC;
   static_assert(CHUNKS % (THREADS * kPair) == 0, "whole rounds");
   const int M = args.M, N = args.N;
   const uint32_t plane = static_cast<uint32_t>(M) * static_cast<uint32_t>(N);
@@ -220,12 +218,12 @@ __device__ __forceinline__ void direct_sum_splits(const DirectArgs& args, int m0
       const int c = c0 + static_cast<int>(threadIdx.x);
       int row, tc;  // row and column in the tile
       if (swiglu) {
-        constexpr int per_row = kDirectBN / 2 / VEC;
+        constexpr int per_row = BN / 2 / VEC;
         row = c / per_row;
         const int g = VEC * (c % per_row);
         tc = g / kSwigluBlock * 2 * kSwigluBlock + g % kSwigluBlock + u * kSwigluBlock;
       } else {
-        constexpr int per_row = kDirectBN / VEC;
+        constexpr int per_row = BN / VEC;
         const int cc = c0 * kPair + u * THREADS + static_cast<int>(threadIdx.x);
         row = cc / per_row;
         tc = VEC * (cc % per_row);
@@ -234,7 +232,7 @@ __device__ __forceinline__ void direct_sum_splits(const DirectArgs& args, int m0
       gn[u] = n0 + tc;
       const bool in = gm < M && gn[u] < N;
       off[u] = in ? (static_cast<uint32_t>(gm) * N + gn[u]) * 4u : kOutOfRange;
-      const uint32_t ocol = swiglu ? n0 / 2 + VEC * (c % (kDirectBN / 2 / VEC)) : gn[u];
+      const uint32_t ocol = swiglu ? n0 / 2 + VEC * (c % (BN / 2 / VEC)) : gn[u];
       dst[u] = in ? (static_cast<uint32_t>(row) * (swiglu ? N / 2 : N) + ocol) * 2u : kOutOfRange;
     }
     vec s[kPair] = {};
@@ -277,28 +275,30 @@ __device__ __forceinline__ void direct_sum_splits(const DirectArgs& args, int m0
   }
 }
 
-// One (32 TM) x 256 output tile (and K split) per workgroup of KW teams of 4
-// waves.  The teams split the workgroup's K range evenly, each with its own
-// ring; their sums meet in LDS in team order at the end.  Two teams pay for
-// small TM, where one wave per SIMD leaves the decode and the barrier of a
-// step exposed (TM = 2, 256 x 4096 x 4096: 30.2 -> 25.9 us unsplit); a large
-// TM hides them behind its own MFMAs.  Workgroups take tiles in blocks of 8
-// row tiles, eighths of the order to each XCD.
-template <int TM, int KW, int GROUP, int OCC>
-__global__ __launch_bounds__(KW* kDirectWaves * 64, OCC) void gemm_direct_kernel(DirectArgs args) {
-  constexpr int BM = 32 * TM, BUF = BM * kDirectStep, RING = kDirectRing, D = RING - 1;
-  constexpr int THREADS = KW * kDirectWaves * 64;
-  constexpr int COPIES = TM;       // 1 KiB copies per wave and step
+// One (32 TM) x (64 WN) output tile (and K split) per workgroup of KW teams of
+// WN waves.  The teams split the workgroup's K range evenly, each with its own
+// ring; their sums meet in LDS in team order at the end.  Teams pay for small
+// batches: the CUs are filled with narrow tiles instead of K splits, whose
+// partials cross HBM, and a second wave per SIMD hides a step's decode and
+// barrier (256 x 4096 x 4096, us: TM = 2, WN = 4 with one team 29.3, with two
+// 25.1; TM = 1, WN = 2 with four 14.9).  A large TM hides them behind its own
+// MFMAs and reads each activation for 256 columns.  Workgroups take tiles in
+// blocks of 8 row tiles, eighths of the order to each XCD.
+template <int TM, int KW, int WN, int GROUP, int OCC>
+__global__ __launch_bounds__(KW* WN * 64, OCC) void gemm_direct_kernel(DirectArgs args) {
+  constexpr int BM = 32 * TM, BN = 64 * WN, BUF = BM * kDirectStep, RING = kDirectRing, D = RING - 1;
+  constexpr int THREADS = KW * WN * 64;
+  constexpr int COPIES = BM / 8 / WN;  // 1 KiB copies per wave and step
   constexpr int LOADS = COPIES + 5;  // and 4 word loads, 1 scale load
   static_assert(GROUP % kDirectStep == 0, "one scale per column per step");
   static_assert((D - 2) * LOADS + 10 + COPIES / 4 <= 63, "vmcnt range");
-  static_assert(KW == 1 || BM * kDirectBN * 4 <= KW * RING * BUF * 2, "team sums fit the rings");
+  static_assert(KW == 1 || BM * BN * 4 <= KW * RING * BUF * 2, "team sums fit the rings");
   __shared__ __attribute__((aligned(16))) _Float16 lds[KW * RING * BUF];
   __shared__ int s_last;
   const int M = args.M, K = args.K, N = args.N;
   const int lane = static_cast<int>(threadIdx.x) & 63;
   const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const int team = KW == 1 ? 0 : wid / kDirectWaves, wave = wid % kDirectWaves;
+  const int team = KW == 1 ? 0 : wid / WN, wave = wid % WN;
   _Float16* const As = lds + team * RING * BUF;
   const uint32_t as_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) void*)As));
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(KW* kDirectWaves * 64, OCC) void gemm_direct_kernel
                                args.tiles_m - block * kDirectGroupM);
   const int tile_n = static_cast<int>(in_block / rows_in);
   const int tile_m = static_cast<int>(block * kDirectGroupM + in_block - tile_n * rows_in);
-  const int m0 = tile_m * BM, n0 = tile_n * kDirectBN;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   // The split's steps, shared out to the teams (the first may take one more).
   const int first = split * args.steps_per_split;
@@ -609,9 +609,9 @@ __global__ __launch_bounds__(KW* kDirectWaves * 64, OCC) void gemm_direct_kernel
   __syncthreads();
   if (!s_last) return;
   if (N % 4 == 0)
-    direct_sum_splits<THREADS, BM, 4>(args, m0, n0);
+    direct_sum_splits<THREADS, BM, BN, 4>(args, m0, n0);
   else
-    direct_sum_splits<THREADS, BM, 2>(args, m0, n0);
+    direct_sum_splits<THREADS, BM, BN, 2>(args, m0, n0);
   if (threadIdx.x == 0)
     __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

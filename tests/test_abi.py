@@ -501,14 +501,14 @@ def test_gemm_fused_validation():
     assert not ext.gemm_fuses(8, 512, 256, 128) and ext.gemm_fuses(32, 4096, 4096, 128)
     assert not ext.gemm_fuses(256, 512, 255, 128) and not ext.gemm_fuses(256, 500, 256, 128)
     assert not ext.gemm_fuses(256, 512, 256, 32) and ext.gemm_fuses(256, 512, 256, 128)
-    assert not ext.gemm_fuses(129, 4096, 4096, 128)  # 64 x 128 tiles, which have no epilogue
+    assert ext.gemm_fuses(129, 4096, 4096, 128)
     for kwargs, needle in ((dict(xc=256), "disagree"), (dict(g=32), "group_size"), (dict(ep=0), "epilogue"),
                            (dict(ep=2, N=272), "multiple of 32"), (dict(bias=None), "bias"),
                            (dict(sw=48), "strip_cols"), (dict(sw=64, N=288), "multiple of strip_cols"),
                            (dict(ptr=None), "null")):
         assert call(**kwargs) == INVALID, kwargs
         assert needle in ext.last_error(), (kwargs, ext.last_error())
-    assert call(M=129, xc=4096, K=4096, N=4096) not in (0, INVALID)
+    assert call(M=8) not in (0, INVALID)  # the decode entry's batches
     assert "no fused epilogue" in ext.last_error()
     assert call(M=0) == 0
 
