@@ -581,7 +581,7 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
   };
   static constexpr Cfg kCfgs[] = {
       {1, 4, 2, 0.127, 0.75}, {2, 4, 2, 0.155, 1.0}, {3, 2, 2, 0.215, 1.0}, {4, 2, 2, 0.275, 1.0},
-      {2, 2, 4, 0.31, 1.0},   {3, 2, 4, 0.37, 1.0},  {1, 1, 4, 0.36, 0.5},  {2, 1, 4, 0.40, 0.5},
+      {2, 2, 4, 0.31, 1.0},   {3, 2, 4, 0.42, 1.0},  {1, 1, 4, 0.36, 0.5},  {2, 1, 4, 0.40, 0.5},
       {3, 1, 4, 0.45, 0.5},   {4, 1, 4, 0.52, 0.5},  {5, 1, 4, 0.68, 1.0},  {6, 1, 4, 0.80, 1.0},
       {8, 1, 4, 1.03, 1.0}};
   const int64_t steps = K / kDirectStep;
