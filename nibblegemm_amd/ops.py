@@ -283,8 +283,9 @@ def gemv(X: torch.Tensor, qw: QuantizedWeight, version: int = 4, splits: int = 0
 
 def gemm(X: torch.Tensor, qw: QuantizedWeight, version: int = 6) -> torch.Tensor:
     """Prefill-regime matmul on MFMA (reference ops.py:77-86).  ``version`` 6
-    (default) or 7 select two tile shapes with identical numerics; batches of
-    M <= 128 run the GEMV's weight-streaming kernel whatever the version.  A
+    (default) or 7, with identical numerics: the plan depends on the sizes
+    only.  Small batches run the GEMV's weight-streaming kernels (up to 32
+    rows, and up to 128 over weights small enough), larger ones tiles.  A
     :class:`StripMajorWeight` runs the same plans and kernels (the same bits
     as its packed weight) from 9 rows, the strip-major GEMV below."""
     if isinstance(qw, StripMajorWeight):
@@ -518,10 +519,17 @@ def _gemm_fused(X: torch.Tensor, qw, epilogue: int, bias: Optional[torch.Tensor]
 
 
 def _tracked(t: torch.Tensor) -> bool:
-    """Whether autograd (reverse or forward mode) follows operations on ``t``:
-    those of a bias stay separate operations, which it records."""
+    """Whether something follows operations on ``t`` -- autograd (reverse or
+    forward mode), a functorch transform, a dispatch or function mode, a
+    tracer, a tensor subclass: a bias is then added as a separate operation,
+    which it sees."""
     return ((t.requires_grad and torch.is_grad_enabled())
-            or torch.autograd.forward_ad._current_level >= 0)
+            or torch.autograd.forward_ad._current_level >= 0
+            or type(t) not in (torch.Tensor, torch.nn.Parameter)
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0
+            or torch.jit.is_tracing())
 
 
 def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> torch.Tensor:

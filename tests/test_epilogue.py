@@ -209,3 +209,26 @@ def test_bias_gradients_still_flow():
     assert torch.allclose(bias.grad.float(), torch.full((N,), float(M), device="cuda"))
     with torch.no_grad():
         assert torch.equal(ng.matmul_bias(Xd, qw, bias), y.detach())
+
+
+def test_bias_under_vmap_and_modes():
+    """A batch of biases, and a bias watched by a dispatch mode, are added as
+    separate ops too."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    M, K, N = 160, 256, 64
+    _, _, _, Xd, qw = synthetic(M, K, N, 128, seed=3)
+    biases = torch.randn(3, N, device="cuda", dtype=torch.float16)
+    y = ng.matmul(Xd, qw)
+    got = torch.vmap(lambda b: ng.matmul_bias(Xd, qw, b))(biases)
+    assert torch.equal(got, y + biases[:, None])
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.overloadpacket._qualified_op_name)
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        watched = ng.matmul_bias(Xd, qw, biases[0])
+    assert "aten::add" in seen and torch.equal(watched, y + biases[0])
