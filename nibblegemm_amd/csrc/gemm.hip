@@ -561,29 +561,37 @@ bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
 
 // The direct kernel's tile, teams and splits for a shape, within the splits
 // and counters of `room`.  A model of its time, fitted to MI355X measurements
-// of every tile and split at some 40 shapes (M = 33..4096), us: 4.5 to start
-// and drain; per 64-k step and round of the CUs the tile's own time, `step`;
-// 0.36 of the time the whole product takes at the power-limited 1.25 PFLOP/s;
-// and for a K split 2 plus its partials at 2 TB/s.  `tail` is how much of a
-// part-filled last round is paid for (less where two workgroups share a CU).
-// It names the fastest plan at most of them and one within ~7% at the rest:
+// of every tile and split at some 45 shapes (M = 33..4096), us: 4.5 to start
+// and drain; per 64-k step and round of the CUs the tile's own time, `step`
+// in a single round and `again` over several; 0.36 of the time the whole
+// product takes at the power-limited 1.25 PFLOP/s; and for a K split 2 plus
+// its partials at 2 TB/s.  `tail` is how much of a part-filled last round is
+// paid for (less where two workgroups share a CU).  Teams are for grids of
+// one round: alone on its CU, such a workgroup's ring fill and the teams'
+// meeting overlap with nothing, so over several rounds its steps take up to
+// half as long again.  The model names the fastest plan at most of the shapes
+// and one within ~7% at the rest:
 // 96 x 8192 x 8192 (M x K x N) tm = 2, 4 teams, 2 columns waves, 2 splits
 // 23.2 us (tm = 1, 2 teams, 4 column waves 26.9), 128 x 4096 x 14336 the same
 // unsplit 19.0 (25.2), 256 x 4096 x 4096 tm = 1, 4 teams 14.9 (2 teams, 2
 // splits 21.8), 512 x 4096 x 14336 tm = 4 52.5 (2: 61, 8: 75), 1000 x 5504 x
-// 4102 tm = 3, 2 teams 48 (4: 54), 3000 x 3072 x 3008 tm = 5 54 (3: 57, 4:
-// 66), 4096 x 4096 x 4096 tm = 8 108 (4: 111).
+// 4102 tm = 3, 2 teams 48 (4: 54), 4096 x 4096 x 4096 tm = 8 108 (4: 111).
+// Several rounds, the fastest tiles without teams against the fastest with:
+// 700 x 4096 x 14336 tm = 6 80 (85), 1024 x 4096 x 28672 tm = 8 198 (222),
+// 1024 x 4096 x 6144 tm = 4 52 (62), 2048 x 5504 x 4102 tm = 5 87 (104), 2048
+// x 4096 x 14336 tm = 5 200 (222).
 // Teams split K, so a K below 1024 keeps one.
 TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, int* splits) {
   struct Cfg {
     int tm, kw, wn;
-    double step, tail;
+    double step, again, tail;
   };
   static constexpr Cfg kCfgs[] = {
-      {1, 4, 2, 0.127, 0.75}, {2, 4, 2, 0.155, 1.0}, {3, 2, 2, 0.215, 1.0}, {4, 2, 2, 0.275, 1.0},
-      {2, 2, 4, 0.31, 1.0},   {3, 2, 4, 0.42, 1.0},  {1, 1, 4, 0.36, 0.5},  {2, 1, 4, 0.40, 0.5},
-      {3, 1, 4, 0.45, 0.5},   {4, 1, 4, 0.52, 0.5},  {5, 1, 4, 0.68, 1.0},  {6, 1, 4, 0.80, 1.0},
-      {8, 1, 4, 1.03, 1.0}};
+      {1, 4, 2, 0.127, 0.127, 0.75}, {2, 4, 2, 0.155, 0.24, 1.0}, {3, 2, 2, 0.215, 0.29, 1.0},
+      {4, 2, 2, 0.275, 0.345, 1.0},  {2, 2, 4, 0.31, 0.36, 1.0},  {3, 2, 4, 0.385, 0.435, 1.0},
+      {1, 1, 4, 0.36, 0.36, 0.5},    {2, 1, 4, 0.40, 0.40, 0.5},  {3, 1, 4, 0.45, 0.45, 0.5},
+      {4, 1, 4, 0.515, 0.515, 0.8},  {5, 1, 4, 0.65, 0.65, 1.0},  {6, 1, 4, 0.775, 0.775, 1.0},
+      {8, 1, 4, 0.98, 0.98, 1.0}};
   const int64_t steps = K / kDirectStep;
   const int64_t max_counters = static_cast<int64_t>(room.counter_bytes / 4);
   const double power = 0.36 * 2.0 * static_cast<double>(M) * K * N / 1.25e9;
@@ -599,7 +607,7 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
       const double fill = static_cast<double>(tiles * s) / kPlanCUs;
       const double rounds = static_cast<double>(ceil_div(tiles * s, kPlanCUs));
       const double eff = fill > 1 ? c.tail * rounds + (1.0 - c.tail) * fill : rounds;
-      double us = 4.5 + eff * static_cast<double>(per) * c.step + power;
+      double us = 4.5 + eff * static_cast<double>(per) * (fill > 1 ? c.again : c.step) + power;
       if (s > 1) us += 2.0 + static_cast<double>(s) * M * N * 4 / 2.0e6;
       if (us < best_us) {
         best_us = us;

@@ -536,7 +536,8 @@ def test_direct_kernel_edges(M, N, K_, g):
 @pytest.mark.parametrize("M,K_,N,g", [(1000, 5504, 4102, 64), (2048, 1344, 6016, 64),
                                       (1024, 4416, 14336, 64), (3000, 3072, 3008, 128),
                                       (1536, 14336, 4096, 128), (300, 8256, 1030, 64),
-                                      (66, 8192, 8196, 128)])
+                                      (66, 8192, 8196, 128), (700, 1088, 14336, 64),
+                                      (256, 4160, 14336, 64), (250, 14336, 4096, 128)])
 def test_direct_kernel_full_grids(M, K_, N, g):
     """Grids that fill the CUs (every tile height the plan picks, K splits,
     K / 64 not a multiple of the ring): every output, and identical bits over
