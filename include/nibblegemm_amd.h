@@ -151,11 +151,11 @@ NIBBLE_API int nibble_gemv_timeline(void* stamps, int64_t bytes);
 
 /*
  * Prefill-regime matmul on CDNA4 MFMA (any M >= 1).  version 6 (default) or 7
- * (alternate tile shape; same numerics).  Requires K % 32 == 0, N even,
+ * (same numerics).  Requires K % 32 == 0, N even,
  * group_size in {64, 128} and M*N, M*K, K*N < 2^31 (the reference's checks).
- * Batches of M <= 128 (with N % 4 == 0) run the weight-streaming kernel of
- * the GEMV, larger ones the tile kernel; either may split K across
- * workgroups.  `workspace` follows the same rules as for nibble_gemv_w4a16,
+ * Small batches (with N % 4 == 0) run the weight-streaming kernels of the
+ * GEMV where nibble_gemm_streams says so, larger ones tiles; either may split
+ * K across workgroups.  `workspace` follows the same rules as for nibble_gemv_w4a16,
  * sized by nibble_gemm_workspace_bytes(...) (NULL allowed when that is 0).
  */
 NIBBLE_API int nibble_gemm_w4a16(const void* X, int64_t x_rows, int64_t x_cols,
@@ -188,7 +188,8 @@ NIBBLE_API int nibble_gemm_streams(int64_t M, int64_t K, int64_t N, int64_t grou
  * followed by the separate ops, to the bit.  `strip_cols` 0 reads packed
  * weights, else strip-major ones of that width.  Workspace as
  * nibble_gemm_workspace_bytes(M, K, N, group_size, 6).  nibble_gemm_fuses: 1
- * where this entry serves these sizes (operands 16-byte aligned), else it returns NIBBLE_ERR_UNSUPPORTED.  ABI version 15. */
+ * where this entry serves these sizes (operands 16-byte aligned), else it
+ * returns NIBBLE_ERR_UNSUPPORTED.  ABI version 15. */
 NIBBLE_API int nibble_gemm_fuses(int64_t M, int64_t K, int64_t N, int64_t group_size);
 NIBBLE_API int nibble_gemm_w4a16_fused(const void* X, int64_t x_rows, int64_t x_cols,
                         const void* Wq, const void* S, int64_t K, int64_t N,

@@ -292,7 +292,7 @@ def attention(args, rows):
             raise RuntimeError(f"attention pos={pos}: max|y - ref| = {err:.3e} * rms(ref)")
         t = H.bench_graph(lambda i: attention_decode(qkv, kcs[i % layers], vcs[i % layers], pos,
                                                      (cos, sin)), reps=32, trials=args.trials)
-        _emit(rows, {"bench": "attention", "pos": pos, "chunks": (pos + 128) // 128,
+        _emit(rows, {"bench": "attention", "pos": pos,
                      "us": round(t.median_ms * 1e3, 2),
                      "kv_GB/s": round(H.achieved_gbps(attention_bytes(n_kv, pos), t.median_ms)),
                      "max_err_rms": float(f"{err:.2e}"), **_clock(t)})

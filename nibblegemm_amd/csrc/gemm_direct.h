@@ -24,10 +24,10 @@
 //     reads of the step before, whose buffer the next loads overwrite.  No
 //     wave drains its LDS reads for it.
 // Measured on MI355X against the kernel this replaced (producer / consumer
-// waves, decoded B through LDS; same bits), us: 512 x 4096 x 14336 (M x K x N)
-// 69 -> 51.5, 2048 x 4096 x 14336 245 -> 190, 2048 x 4096 x 28672 480 -> 378,
-// 2048 x 14336 x 4096 235 -> 193 (1.25 PFLOP/s; hipBLASLt's fp16 product
-// 220).  What it took: loads spread over the slices instead of one burst a
+// waves, decoded B through LDS; same bits), weights from HBM, us: 512 x 4096 x
+// 14336 (M x K x N) 71 -> 54.5, 2048 x 4096 x 14336 248 -> 197 (1.22 PFLOP/s;
+// hipBLASLt's fp16 product 200), 2048 x 14336 x 4096 234 -> 193 (1.25; 216),
+// 4096 x 14336 x 4096 440 -> 359 (1.34; 346).  What it took: loads spread over the slices instead of one burst a
 // step, and the barrier without an LDS drain (one deeper ring), 212 -> 193 at
 // 2048 x 14336 x 4096; the B words in LDS or three ring buffers lose.
 #pragma once

@@ -1375,11 +1375,11 @@ constexpr int kBatchStagers = 4;
 constexpr int kBatchWorkgroups = 256;
 constexpr int kBatchMaxSplits = 8;
 // 33..64 rows run one 64-row block only when its grid fills the CUs in one
-// round (224..256 workgroups).  Measured on MI355X against gemm's 64-row
-// tiles, M = 33 / 64: 4096 x 14336 17.1 / 17.6 us against 19.2 / 19.7,
-// 14336 x 4096 17.4 / 18.8 against 20.0 / 21.6, 4096 x 4096 11.0 / 11.0
-// against 11.9 / 12.4; 192 workgroups (4096 x 6144) 12.9 against 12.3, two
-// rounds (4096 x 28672) 29.9 against 26.2.
+// round (224..256 workgroups).  Measured on MI355X, M = 33 / 64: 4096 x 14336
+// 14.9 / 15.7 us (the GEMM's tiles 17.2 at 65 rows).  Against the tiles before
+// the direct kernel: 14336 x 4096 17.4 / 18.8 us and 20.0 / 21.6, 4096 x 4096
+// 11.0 / 11.0 and 11.9 / 12.4; 192 workgroups (4096 x 6144) 12.9 and 12.3, two
+// rounds (4096 x 28672) 29.9 and 26.2.
 constexpr int kBatch64MinWorkgroups = 224;
 // 16-row blocks run the batch kernel from this many rows: at 9 rows the
 // split kernel, whose activation loads scale with the rows, is as fast or

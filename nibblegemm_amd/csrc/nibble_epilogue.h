@@ -1,7 +1,7 @@
-// Output epilogues of the weight-streaming kernels: fused forms of what a
-// caller would otherwise run as separate elementwise ops on the fp16 product.
-// Shared by the decode GEMV (gemv.hip) and the persistent decode chain
-// (chain.hip), which must give the same bits.
+// Output epilogues of the matmul kernels: fused forms of what a caller would
+// otherwise run as separate elementwise ops on the fp16 product.  Shared by
+// the decode GEMV (gemv.hip), the persistent decode chain (chain.hip) and the
+// prefill GEMM (gemm_direct.h), which must give the same bits.
 #pragma once
 
 #include <hip/hip_runtime.h>
