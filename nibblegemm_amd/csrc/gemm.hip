@@ -943,6 +943,9 @@ extern "C" int nibble_gemm_w4a16_fused(const void* X, int64_t x_rows, int64_t x_
                "strip_cols must be 0 (packed), 16, 32 or 64, got %lld", (long long)strip_cols);
   NIBBLE_CHECK(strip_cols == 0 || N % strip_cols == 0, "N=%lld is not a multiple of strip_cols=%lld",
                (long long)N, (long long)strip_cols);
+  NIBBLE_CHECK(strip_cols != 16 || group_size == 128, "16-column strips need group_size 128");
+  NIBBLE_CHECK(strip_cols == 0 || Wq == nullptr || (aligned(Wq, 16) && aligned(S, 16)),
+               "strip-major weights and scales must be 16-byte aligned");
   NIBBLE_CHECK(epilogue == kEpilogueBias || epilogue == kEpilogueSwiglu,
                "epilogue must be 1 (bias) or 2 (swiglu), got %lld", (long long)epilogue);
   NIBBLE_CHECK(epilogue != kEpilogueSwiglu || N % (2 * kSwigluBlock) == 0,

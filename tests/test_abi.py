@@ -495,8 +495,8 @@ def test_gemm_fused_validation():
     other tiles and epilogues, mismatched shapes, missing biases."""
     ext = ng.extension()
 
-    def call(M=256, xc=512, K=512, N=256, g=128, sw=0, ep=1, bias=P, ptr=P):
-        return ext.gemm_fused(ptr, M, xc, ptr, ptr, K, N, g, sw, ep, bias, ptr, None, 0, None)
+    def call(M=256, xc=512, K=512, N=256, g=128, sw=0, ep=1, bias=P, ptr=P, w=None):
+        return ext.gemm_fused(ptr, M, xc, w or ptr, ptr, K, N, g, sw, ep, bias, ptr, None, 0, None)
 
     assert not ext.gemm_fuses(8, 512, 256, 128) and ext.gemm_fuses(32, 4096, 4096, 128)
     assert not ext.gemm_fuses(256, 512, 255, 128) and not ext.gemm_fuses(256, 500, 256, 128)
@@ -505,6 +505,7 @@ def test_gemm_fused_validation():
     for kwargs, needle in ((dict(xc=256), "disagree"), (dict(g=32), "group_size"), (dict(ep=0), "epilogue"),
                            (dict(ep=2, N=272), "multiple of 32"), (dict(bias=None), "bias"),
                            (dict(sw=48), "strip_cols"), (dict(sw=64, N=288), "multiple of strip_cols"),
+                           (dict(sw=16, g=64), "group_size 128"), (dict(sw=32, w=P + 8), "16-byte aligned"),
                            (dict(ptr=None), "null")):
         assert call(**kwargs) == INVALID, kwargs
         assert needle in ext.last_error(), (kwargs, ext.last_error())
