@@ -580,7 +580,10 @@ bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
 // 700 x 4096 x 14336 tm = 6 80 (85), 1024 x 4096 x 28672 tm = 8 198 (222),
 // 1024 x 4096 x 6144 tm = 4 52 (62), 2048 x 5504 x 4102 tm = 5 87 (104), 2048
 // x 4096 x 14336 tm = 5 200 (222).
-// Teams split K, so a K below 1024 keeps one.
+// Teams split K, so a K below 1024 keeps one, except from 512 where 32-row
+// tiles make one round: 129 / 300 x 768 x 3072 8.0 / 8.3 us with one team, 6.4
+// / 6.7 with four; 129 / 256 x 512 x 4096 6.4 / 6.7, 5.9 / 6.1.  Beyond a
+// round 64-row tiles with teams lose: 300 x 512 x 4096 6.8, 7.5.
 TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, int* splits) {
   struct Cfg {
     int tm, kw, wn;
@@ -598,8 +601,9 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
   TileChoice best{0, 0};
   double best_us = 1e30;
   for (const Cfg& c : kCfgs) {
-    if (c.kw > 1 ? K < 1024 : c.tm <= 3 && K >= 1024) continue;
     const int64_t tiles = ceil_div(M, 32 * c.tm) * ceil_div(N, 64 * c.wn);
+    const bool teams = K >= 1024 || (K >= 512 && c.tm == 1 && tiles <= kPlanCUs);
+    if (c.kw > 1 ? !teams : c.tm <= 3 && K >= 1024) continue;
     for (int s = 1; s <= (c.tm <= kDirectMaxSplitTM ? room.splits : 1); ++s) {
       if (s > 1 && tiles > max_counters) break;
       const int64_t per = ceil_div(steps, s);

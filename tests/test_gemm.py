@@ -513,12 +513,13 @@ def test_split_k_sum_into_under_aligned_output():
         buf.zero_()
 
 
-@pytest.mark.parametrize("K_,g", [(64, 64), (128, 128), (192, 64), (320, 64), (2048, 128), (2176, 64),
-                                  (2240, 64), (2304, 128), (4288, 64)])
+@pytest.mark.parametrize("K_,g", [(64, 64), (128, 128), (192, 64), (320, 64), (512, 128), (576, 64),
+                                  (832, 64), (2048, 128), (2176, 64), (2240, 64), (2304, 128),
+                                  (4288, 64)])
 @pytest.mark.parametrize("M,N", [(33, 258), (129, 254), (191, 1030), (256, 512), (700, 514)])
 def test_direct_kernel_edges(M, N, K_, g):
     """The direct kernel's tails: every remainder of its 4-step rings (one to
-    five 64-k steps, and with two teams from K = 2048 uneven team shares), row
+    five 64-k steps, and with teams from K = 512 uneven shares or none), row
     tiles and 256-column tiles cut anywhere, N only even, both group sizes.
     Every output against an fp32 product of the dequant kernel's weights; a
     step multiplied before its activations had landed would be a whole step
