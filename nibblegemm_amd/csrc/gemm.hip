@@ -623,11 +623,14 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
   return best;
 }
 
-// The launch plan.  `direct` says the operands suit the direct kernel.  Both
-// versions take the same plan wherever their workspaces agree, so they agree
-// to the bit.
+// The launch plan.  `direct` says the operands suit the direct kernel, which
+// loads two columns at a time whatever more their alignment allows (bn_max):
+// its room is the workspace query's, so the splits, the workspace they need
+// and where the counters end are what the caller was told.  Both versions
+// take the same plan wherever their workspaces agree, and then agree to the
+// bit.
 TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max, bool direct) {
-  TilePlan p = plan_split_room(M, K, N, version, bn_max);
+  TilePlan p = plan_split_room(M, K, N, version, direct ? nominal_bn_max(N) : bn_max);
   if (direct) {
     int splits = 1;
     p.t = choose_direct(M, K, N, p, &splits);

@@ -459,6 +459,33 @@ def test_gemm_under_aligned_weights(M, K_, N):
     assert rms_err(host(y_off), oracle_y(X, packed, scales, K_, 128)) <= RMS_TOL
 
 
+@pytest.mark.parametrize("words,scale", [(2, 2), (2, 0), (0, 2)])
+@pytest.mark.parametrize("M,K_,N", [(96, 8192, 8192), (384, 14336, 4096), (129, 8192, 4096)])
+def test_split_plans_under_aligned_weights(M, K_, N, words, scale):
+    """Weights 8-byte and scales 4-byte aligned run the aligned call's plan with
+    its K splits, in the workspace that the query reports: the same bits."""
+    ext = ng.extension()
+    ws_bytes, counter_bytes = ext.gemm_workspace_bytes(M, K_, N, 128, 6, None)
+    assert counter_bytes > 0  # this plan splits K
+    _, _, _, Xd, qw = synthetic(M, K_, N, 128, seed=M + N)
+    qw_off = ng.QuantizedWeight(_offset_copy(qw.qweight, words), _offset_copy(qw.scales, scale),
+                                128, K_, N)
+    assert qw_off.qweight.data_ptr() % 16 == 4 * words and qw_off.scales.data_ptr() % 8 == 2 * scale
+    y = ng.gemm(Xd, qw)
+    ws = torch.zeros(ws_bytes + 512, dtype=torch.uint8, device=Xd.device)
+    ws[ws_bytes:] = 0xA5  # what follows the reported workspace stays as it was
+    out = torch.empty_like(y)
+    for _ in range(3):  # the counters return to zero
+        rc = ext.gemm(Xd.data_ptr(), M, K_, qw_off.qweight.data_ptr(), K_ // 8, N,
+                      qw_off.scales.data_ptr(), K_ // 128, N, 128, 6, out.data_ptr(),
+                      ws.data_ptr(), ws_bytes, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, ext.last_error()
+        assert torch.equal(out, y)
+    assert ws[:counter_bytes].eq(0).all() and ws[ws_bytes:].eq(0xA5).all()
+    ng.ops.release_workspaces()
+    assert torch.equal(ng.gemm(Xd, qw_off), y)
+
+
 @pytest.mark.parametrize("M,K_,N", [(160, 14336, 512), (64, 14336, 4096), (129, 4096, 4096)])
 def test_split_k_gemm_replays_in_a_graph(M, K_, N):
     """The producer/consumer kernel's K split (counters reset by the kernel
