@@ -30,6 +30,9 @@ import threading
 from typing import Dict, Optional, Tuple
 
 import torch
+from torch import _C
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _native
 from .quant import (SWIGLU_BLOCK, QuantizedWeight, StripMajorWeight,  # noqa: F401
@@ -522,13 +525,21 @@ def _tracked(t: torch.Tensor) -> bool:
     """Whether something follows operations on ``t`` -- autograd (reverse or
     forward mode), a functorch transform, a dispatch or function mode, a
     tracer, a tensor subclass: a bias is then added as a separate operation,
-    which it sees."""
+    which it sees.  A default device (``torch.set_default_device``) is a
+    function mode too, but follows factory calls only."""
     return ((t.requires_grad and torch.is_grad_enabled())
-            or torch.autograd.forward_ad._current_level >= 0
             or type(t) not in (torch.Tensor, torch.nn.Parameter)
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._len_torch_function_stack() > 0
+            or forward_ad._current_level >= 0 or _modes_follow())
+
+
+def _modes_follow() -> bool:
+    """Whether a functorch transform, a dispatch mode, a function mode that is
+    not a default device, or a tracer is active."""
+    functions = _C._len_torch_function_stack()
+    return (_C._functorch.peek_interpreter_stack() is not None
+            or _C._len_torch_dispatch_stack() > 0
+            or (functions > 0 and any(type(_C._get_function_stack_at(i)) is not DeviceContext
+                                      for i in range(functions)))
             or torch.jit.is_tracing())
 
 
@@ -537,16 +548,17 @@ def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> tor
     ``QuantLinear`` with a bias (ops.py:131-135): the fp16 product, then the
     bias added in fp16.  An fp16 bias runs as one launch (the bias added in
     the kernel's epilogue, same bits) wherever the kernel the product runs on
-    has one; other cases run the two ops."""
+    has one; other cases, and a bias that something follows
+    (:func:`_tracked`), run the two ops."""
     _check_2d(X, qw)
     fp16_bias = (bias.dtype == torch.float16 and bias.dim() == 1 and bias.numel() == qw.N
-                 and bias.device == X.device and bias.is_contiguous())
+                 and bias.device == X.device and bias.is_contiguous() and not _tracked(bias))
     if isinstance(qw, StripMajorWeight):
         if fp16_bias and X.size(0) <= DECODE_MAX_M:
             return _strip_gemv(X, qw, 1, bias, qw.N)
     elif fp16_bias and _fusable(X, qw):
         return _fused(X, qw, 1, bias, qw.N)
-    if fp16_bias and not _tracked(bias) and _gemm_fusable(X, qw):
+    if fp16_bias and _gemm_fusable(X, qw):
         return _gemm_fused(X, qw, 1, bias, qw.N)
     return matmul(X, qw) + bias
 
@@ -614,7 +626,7 @@ def rmsnorm_matmul(X: torch.Tensor, norm_weight: torch.Tensor, qw: QuantizedWeig
             and norm_weight.data_ptr() % 16 == 0 and X.dtype == torch.float16
             and (bias is None or (bias.dtype == torch.float16 and bias.dim() == 1
                                   and bias.numel() == qw.N and bias.is_contiguous()
-                                  and bias.device == X.device))):
+                                  and bias.device == X.device and not _tracked(bias)))):
         run = _strip_gemv if strip else _fused
         if swiglu:
             return run(X, qw, 2, None, qw.N // 2, (norm_weight, eps))

@@ -199,25 +199,37 @@ def test_gemm_swiglu_of_extreme_products():
     assert torch.equal(got.nan_to_num(nan=1.0), want.nan_to_num(nan=1.0))
 
 
-def test_bias_gradients_still_flow():
-    """A bias that autograd follows is added as a separate op."""
-    M, K, N = 160, 256, 64
+@pytest.mark.parametrize("layout", ["packed", "strip"])
+@pytest.mark.parametrize("M", [1, 3, 16, 100, 160])
+def test_bias_gradients_still_flow(M, layout):
+    """A bias that autograd follows is added as a separate op, whatever kernel
+    the product runs on; so is it behind a fused RMSNorm."""
+    K, N = 256, 64
     _, _, _, Xd, qw = synthetic(M, K, N, 128, seed=3)
-    bias = torch.randn(N, device="cuda", dtype=torch.float16, requires_grad=True)
-    y = ng.matmul_bias(Xd, qw, bias)
-    y.float().sum().backward()
-    assert torch.allclose(bias.grad.float(), torch.full((N,), float(M), device="cuda"))
-    with torch.no_grad():
-        assert torch.equal(ng.matmul_bias(Xd, qw, bias), y.detach())
+    if layout == "strip":
+        qw = ng.ops.to_strip_major(qw)
+    norm = torch.ones(K, device="cuda", dtype=torch.float16)
+    for call in (ng.matmul_bias, lambda X, w, b: ng.ops.rmsnorm_matmul(X, norm, w, bias=b)):
+        bias = torch.randn(N, device="cuda", dtype=torch.float16, requires_grad=True)
+        y = call(Xd, qw, bias)
+        y.float().sum().backward()
+        assert torch.allclose(bias.grad.float(), torch.full((N,), float(M), device="cuda"))
+        with torch.no_grad():
+            assert torch.equal(call(Xd, qw, bias), y.detach())
 
 
-def test_bias_under_vmap_and_modes():
-    """A batch of biases, and a bias watched by a dispatch mode, are added as
-    separate ops too."""
+@pytest.mark.parametrize("layout", ["packed", "strip"])
+@pytest.mark.parametrize("M", [1, 16, 160])
+def test_bias_under_vmap_and_modes(M, layout):
+    """A batch of biases, and a bias watched by a dispatch or function mode,
+    are added as separate ops too; a default device is no such watcher."""
+    from torch.overrides import TorchFunctionMode
     from torch.utils._python_dispatch import TorchDispatchMode
 
-    M, K, N = 160, 256, 64
+    K, N = 256, 64
     _, _, _, Xd, qw = synthetic(M, K, N, 128, seed=3)
+    if layout == "strip":
+        qw = ng.ops.to_strip_major(qw)
     biases = torch.randn(3, N, device="cuda", dtype=torch.float16)
     y = ng.matmul(Xd, qw)
     got = torch.vmap(lambda b: ng.matmul_bias(Xd, qw, b))(biases)
@@ -232,3 +244,14 @@ def test_bias_under_vmap_and_modes():
     with Mode():
         watched = ng.matmul_bias(Xd, qw, biases[0])
     assert "aten::add" in seen and torch.equal(watched, y + biases[0])
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Functions():
+        watched = ng.matmul_bias(Xd, qw, biases[0])
+    assert torch.Tensor.add in seen and torch.equal(watched, y + biases[0])
+    with torch.device("cuda"):
+        assert not ops._tracked(biases[0])
