@@ -30,13 +30,11 @@ import threading
 from typing import Dict, Optional, Tuple
 
 import torch
-from torch import _C
 from torch.autograd import forward_ad
-from torch.utils._device import DeviceContext
 
 from . import _native
 from .quant import (SWIGLU_BLOCK, QuantizedWeight, StripMajorWeight,  # noqa: F401
-                    from_strip_major, quantize, split_swiglu)
+                    from_strip_major, modes_follow, quantize, split_swiglu)
 
 #: Batch sizes at or below this go to the bandwidth-bound decode kernel
 #: (reference ops.py:30).
@@ -525,22 +523,10 @@ def _tracked(t: torch.Tensor) -> bool:
     """Whether something follows operations on ``t`` -- autograd (reverse or
     forward mode), a functorch transform, a dispatch or function mode, a
     tracer, a tensor subclass: a bias is then added as a separate operation,
-    which it sees.  A default device (``torch.set_default_device``) is a
-    function mode too, but follows factory calls only."""
+    which it sees."""
     return ((t.requires_grad and torch.is_grad_enabled())
             or type(t) not in (torch.Tensor, torch.nn.Parameter)
-            or forward_ad._current_level >= 0 or _modes_follow())
-
-
-def _modes_follow() -> bool:
-    """Whether a functorch transform, a dispatch mode, a function mode that is
-    not a default device, or a tracer is active."""
-    functions = _C._len_torch_function_stack()
-    return (_C._functorch.peek_interpreter_stack() is not None
-            or _C._len_torch_dispatch_stack() > 0
-            or (functions > 0 and any(type(_C._get_function_stack_at(i)) is not DeviceContext
-                                      for i in range(functions)))
-            or torch.jit.is_tracing())
+            or getattr(forward_ad, "_current_level", 0) >= 0 or modes_follow())
 
 
 def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> torch.Tensor:

@@ -30,6 +30,11 @@ from dataclasses import dataclass
 import numpy as np
 import torch
 
+try:
+    from torch.utils._device import DeviceContext as _DeviceContext
+except ImportError:  # then a default device counts as a mode (modes_follow)
+    _DeviceContext = None
+
 #: Nibble slot of each logical k within a packed word.
 SLOT_FOR_K = np.array([0, 4, 1, 5, 2, 6, 3, 7], dtype=np.int64)
 #: Logical k held by each nibble slot (the inverse permutation).
@@ -137,16 +142,32 @@ _KERNEL_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 _KERNEL_MAX_GROUP = 512
 
 
+def modes_follow() -> bool:
+    """Whether a functorch transform, a dispatch or function mode, or a tracer
+    follows torch operations (which would not see a kernel launched beside
+    them).  A default device (``torch.set_default_device``) is a function mode
+    too, but follows factory calls only.  True also where this torch has no
+    such name to ask: operations serve every case."""
+    C = torch._C
+    try:
+        functions = C._len_torch_function_stack()
+        return (C._functorch.peek_interpreter_stack() is not None
+                or C._len_torch_dispatch_stack() > 0
+                or (functions > 0 and any(type(C._get_function_stack_at(i)) is not _DeviceContext
+                                          for i in range(functions)))
+                or torch.jit.is_tracing())
+    except AttributeError:
+        return True
+
+
 def _kernel_quantizes(W: torch.Tensor, group_size: int) -> bool:
     """Whether :func:`quantize_device` runs ``W`` through its kernel: a plain
-    contiguous GPU tensor of a dtype it reads, not one that a tracer, a
-    dispatch mode or a functorch transform wants to see operations on."""
+    contiguous GPU tensor of a dtype it reads, with nothing that follows
+    operations on it (:func:`modes_follow`)."""
     return (W.is_cuda and W.dtype in _KERNEL_DTYPES and W.numel() > 0
             and type(W) in (torch.Tensor, torch.nn.Parameter) and W.is_contiguous()
             and 8 <= group_size <= _KERNEL_MAX_GROUP and W.shape[0] // group_size < 65536
-            and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+            and not torch.compiler.is_compiling() and not modes_follow())
 
 
 def quantize_device(W: torch.Tensor, group_size: int = 128) -> QuantizedWeight:
