@@ -561,17 +561,20 @@ bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
 
 // The direct kernel's tile, teams and splits for a shape, within the splits
 // and counters of `room`.  A model of its time, fitted to MI355X measurements
-// of every tile and split at some 45 shapes (M = 33..4096), us: 4.5 to start
-// and drain; per 64-k step and round of the CUs the tile's own time, `step`
-// in a single round and `again` over several; 0.36 of the time the whole
-// product takes at the power-limited 1.25 PFLOP/s; and for a K split 2 plus
-// its partials at 2 TB/s.  `tail` is how much of a part-filled last round is
-// paid for (less where two workgroups share a CU).  Teams are for grids of
-// one round: alone on its CU, such a workgroup's ring fill and the teams'
-// meeting overlap with nothing, so over several rounds its steps take up to
-// half as long again.  The model names the fastest plan at most of the shapes
-// and one within ~7% at the rest:
-// 96 x 8192 x 8192 (M x K x N) tm = 2, 4 teams, 2 columns waves, 2 splits
+// of every tile and split at some 900 shapes (M = 48..1536) and the fastest
+// tiles beyond, us: 4.5 to start and drain; per 64-k step and round of the CUs
+// the tile's own time, `step` in a single round and `again` over several; 0.36
+// of the time the whole product takes at the power-limited 1.25 PFLOP/s; and
+// for a K split 1 + 0.5 a split, 0.9 for each round of coherent loads the last
+// workgroup of a tile sums it in (4 tm / kw rounds: 3 us for tm = 1, 4 teams;
+// 5 to 10 for tm = 2; 9 to 13 for tm = 3, 2 teams) and 0.26 a MB of partials.
+// `tail` is how much of a part-filled last round is paid for (less where two
+// workgroups share a CU).  Teams are for grids of one round: alone on its CU,
+// such a workgroup's ring fill and the teams' meeting overlap with nothing, so
+// over several rounds its steps take up to half as long again.  The model
+// names the fastest plan at most of the shapes, one within 5% at six of seven
+// and within 10% at nineteen of twenty:
+// 96 x 8192 x 8192 (M x K x N) tm = 2, 4 teams, 2 column waves, 2 splits
 // 23.2 us (tm = 1, 2 teams, 4 column waves 26.9), 128 x 4096 x 14336 the same
 // unsplit 19.0 (25.2), 256 x 4096 x 4096 tm = 1, 4 teams 14.9 (2 teams, 2
 // splits 21.8), 512 x 4096 x 14336 tm = 4 52.5 (2: 61, 8: 75), 1000 x 5504 x
@@ -580,20 +583,28 @@ bool direct_supported(int64_t K, int64_t N, const void* w, const void* s) {
 // 700 x 4096 x 14336 tm = 6 80 (85), 1024 x 4096 x 28672 tm = 8 198 (222),
 // 1024 x 4096 x 6144 tm = 4 52 (62), 2048 x 5504 x 4102 tm = 5 87 (104), 2048
 // x 4096 x 14336 tm = 5 200 (222).
-// Teams split K, so a K below 1024 keeps one, except from 512 where 32-row
-// tiles make one round: 129 / 300 x 768 x 3072 8.0 / 8.3 us with one team, 6.4
-// / 6.7 with four; 129 / 256 x 512 x 4096 6.4 / 6.7, 5.9 / 6.1.  Beyond a
-// round 64-row tiles with teams lose: 300 x 512 x 4096 6.8, 7.5.
+// Tiles of one column wave (64 columns) are for few tiles, where they make one
+// round: a K split of wider tiles costs more than their narrower rows lose.
+// 129 x 4096 x 2048 tm = 1, 4 teams 12.0 (tm = 2, 2 column waves, 4 splits
+// 15.8), 400 x 4096 x 1024 12.4 (18.0), 700 x 4096 x 512 12.3 (14.9), 300 x
+// 8192 x 2048 tm = 2 23.0 (tm = 1, 2 column waves 24.5); over two rounds they
+// lose, 300 x 4096 x 2048 tm = 1 17.0 (15.3).
+// Teams split K, so a K below 1024 keeps one, except from 512 in one round of
+// 32-row tiles, or of 64-row tiles with 2 teams: 300 x 768 x 3072 32-row 6.5 us
+// (one team 8.3), 129 / 256 x 512 x 4096 5.9 / 6.1 (6.4 / 6.7); 400 x 768 x
+// 3072 64-row 7.1 (8.4), 300 x 512 x 4096 6.2 (6.9), and beyond a round 700 x
+// 768 x 3072 9.7 (8.7).
 TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, int* splits) {
   struct Cfg {
     int tm, kw, wn;
     double step, again, tail;
   };
   static constexpr Cfg kCfgs[] = {
-      {1, 4, 2, 0.127, 0.127, 0.75}, {2, 4, 2, 0.155, 0.24, 1.0}, {3, 2, 2, 0.215, 0.29, 1.0},
-      {4, 2, 2, 0.275, 0.345, 1.0},  {2, 2, 4, 0.31, 0.36, 1.0},  {3, 2, 4, 0.385, 0.435, 1.0},
-      {1, 1, 4, 0.36, 0.36, 0.5},    {2, 1, 4, 0.40, 0.40, 0.5},  {3, 1, 4, 0.45, 0.45, 0.5},
-      {4, 1, 4, 0.515, 0.515, 0.8},  {5, 1, 4, 0.65, 0.65, 1.0},  {6, 1, 4, 0.775, 0.775, 1.0},
+      {1, 4, 1, 0.108, 0.108, 1.0},  {2, 4, 1, 0.13, 0.13, 1.0},   {2, 2, 2, 0.165, 0.165, 1.0},
+      {1, 4, 2, 0.127, 0.127, 0.75}, {2, 4, 2, 0.155, 0.24, 1.0},  {3, 2, 2, 0.215, 0.29, 1.0},
+      {4, 2, 2, 0.275, 0.345, 1.0},  {2, 2, 4, 0.28, 0.36, 1.0},   {3, 2, 4, 0.385, 0.435, 1.0},
+      {1, 1, 4, 0.36, 0.36, 0.5},    {2, 1, 4, 0.40, 0.40, 0.5},   {3, 1, 4, 0.45, 0.45, 0.5},
+      {4, 1, 4, 0.515, 0.515, 0.8},  {5, 1, 4, 0.65, 0.65, 1.0},   {6, 1, 4, 0.775, 0.775, 1.0},
       {8, 1, 4, 0.98, 0.98, 1.0}};
   const int64_t steps = K / kDirectStep;
   const int64_t max_counters = static_cast<int64_t>(room.counter_bytes / 4);
@@ -602,8 +613,15 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
   double best_us = 1e30;
   for (const Cfg& c : kCfgs) {
     const int64_t tiles = ceil_div(M, 32 * c.tm) * ceil_div(N, 64 * c.wn);
-    const bool teams = K >= 1024 || (K >= 512 && c.tm == 1 && tiles <= kPlanCUs);
-    if (c.kw > 1 ? !teams : c.tm <= 3 && K >= 1024) continue;
+    const bool one_round = tiles <= kPlanCUs;
+    const bool short_k_form = c.tm == 2 && c.kw == 2 && c.wn == 2;
+    if (c.kw == 1) {
+      if (c.tm <= 3 && K >= 1024) continue;
+    } else if (K < 1024) {
+      if (K < 512 || !one_round || !(c.tm == 1 || short_k_form)) continue;
+    } else if (short_k_form || (c.wn == 1 && !one_round)) {
+      continue;
+    }
     for (int s = 1; s <= (c.tm <= kDirectMaxSplitTM ? room.splits : 1); ++s) {
       if (s > 1 && tiles > max_counters) break;
       const int64_t per = ceil_div(steps, s);
@@ -612,7 +630,8 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
       const double rounds = static_cast<double>(ceil_div(tiles * s, kPlanCUs));
       const double eff = fill > 1 ? c.tail * rounds + (1.0 - c.tail) * fill : rounds;
       double us = 4.5 + eff * static_cast<double>(per) * (fill > 1 ? c.again : c.step) + power;
-      if (s > 1) us += 2.0 + static_cast<double>(s) * M * N * 4 / 2.0e6;
+      if (s > 1)
+        us += 1.0 + 0.5 * s + 0.9 * 4 * c.tm / c.kw + 0.26e-6 * 4 * static_cast<double>(s) * M * N;
       if (us < best_us) {
         best_us = us;
         best = TileChoice{32 * c.tm, 64 * c.wn, c.tm, c.kw, c.wn};
@@ -642,6 +661,9 @@ TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max,
 
 hipError_t launch_direct(TileChoice t, const DirectArgs& a, int64_t G, hipStream_t stream) {
   switch (t.tm * 100 + t.kw * 10 + t.wn) {
+    case 141: return launch_direct_cfg<1, 4, 1>(a, G, stream);
+    case 241: return launch_direct_cfg<2, 4, 1>(a, G, stream);
+    case 222: return launch_direct_cfg<2, 2, 2>(a, G, stream);
     case 142: return launch_direct_cfg<1, 4, 2>(a, G, stream);
     case 242: return launch_direct_cfg<2, 4, 2>(a, G, stream);
     case 322: return launch_direct_cfg<3, 2, 2>(a, G, stream);

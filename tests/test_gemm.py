@@ -578,3 +578,28 @@ def test_direct_kernel_full_grids(M, K_, N, g):
     assert float((ys[0].float() - ref).abs().max() / rms) <= RMS_TOL
     for y in ys[1:]:
         assert torch.equal(y, ys[0])
+
+
+@pytest.mark.parametrize("M,K_,N,g", [
+    (129, 4096, 2048, 128), (400, 4160, 1030, 64), (161, 1088, 2050, 64), (33, 1984, 254, 64),
+    (129, 512, 3070, 128), (130, 4096, 512, 128), (97, 14336, 510, 128),  # 32 x 64 tiles
+    (300, 8256, 2048, 64), (513, 8192, 1026, 128), (129, 14336, 3070, 128),  # 64 x 64 tiles
+    (400, 768, 3072, 128), (513, 576, 2050, 64), (1500, 960, 1022, 64)])  # 64 x 128, two teams
+def test_one_round_tiles(M, K_, N, g):
+    """The tiles that are taken where they make one round of the CUs -- one
+    column wave with four teams, and two teams below K = 1024 -- with row,
+    column and step remainders: every output against an fp32 product of the
+    dequant kernel's weights (the split ones too), 20 calls with the same bits,
+    and the same bits on strip-major weights."""
+    _, _, _, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
+    ref = Xd.float() @ ng.dequant(qw).float()
+    rms = ref.pow(2).mean().sqrt()
+    ys = [ng.gemm(Xd, qw) for _ in range(20)]
+    torch.cuda.synchronize()
+    assert float((ys[0].float() - ref).abs().max() / rms) <= RMS_TOL
+    for y in ys[1:]:
+        assert torch.equal(y, ys[0])
+    if N % 64 == 0:
+        assert torch.equal(ng.gemm(Xd, ng.ops.to_strip_major(qw, 64)), ys[0])
+    bias = torch.randn(N, device="cuda").half()
+    assert torch.equal(ng.matmul_bias(Xd, qw, bias), ys[0] + bias)
