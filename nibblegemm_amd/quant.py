@@ -184,9 +184,10 @@ def quantize_device(W: torch.Tensor, group_size: int = 128) -> QuantizedWeight:
         ext = _native.binding()
         packed = torch.empty((K // PACK_FACTOR, N), dtype=torch.int32, device=W.device)
         scales = torch.empty((K // group_size, N), dtype=torch.float16, device=W.device)
-        rc = ext.quantize_rtn(W.data_ptr(), K, N, _KERNEL_DTYPES[W.dtype], group_size,
-                              packed.data_ptr(), scales.data_ptr(),
-                              torch.cuda.current_stream(W.device).cuda_stream)
+        with torch.cuda.device(W.device):  # a null stream is the current device's
+            rc = ext.quantize_rtn(W.data_ptr(), K, N, _KERNEL_DTYPES[W.dtype], group_size,
+                                  packed.data_ptr(), scales.data_ptr(),
+                                  torch.cuda.current_stream(W.device).cuda_stream)
         if rc:
             raise RuntimeError(f"nibblegemm_amd: {ext.last_error()} (status {rc})")
         return QuantizedWeight(packed, scales, group_size, K, N)

@@ -184,3 +184,37 @@ def test_quantize_with_clip_search_uses_the_searched_scales():
     deq = dequantize(qw).float()
     rtn = dequantize(quantize(W, G)).float()
     assert (deq - W).pow(2).mean() < (rtn - W).pow(2).mean()
+
+
+def test_quantize_device_launches_on_the_weights_device(monkeypatch):
+    """The kernel runs with W's device current: torch's default stream is the
+    null stream, which belongs to whichever device is current.  (The launch
+    itself is replaced; no GPU is needed.)"""
+    import contextlib
+
+    from nibblegemm_amd import _native
+
+    current, launched = [], []
+
+    @contextlib.contextmanager
+    def device(d):
+        current.append(d)
+        yield
+        current.pop()
+
+    class Stub:
+        @staticmethod
+        def quantize_rtn(*args):
+            launched.append((list(current), args[1:5]))
+            return 0
+
+    class Null:
+        cuda_stream = 0
+
+    monkeypatch.setattr(quant, "_kernel_quantizes", lambda W, g: True)
+    monkeypatch.setattr(_native, "binding", lambda: Stub)
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: Null)
+    W = torch.randn(128, 16)
+    quant.quantize_device(W, 64)
+    assert launched == [([W.device], (128, 16, 2, 64))] and not current
