@@ -522,9 +522,9 @@ def _gemm_fused(X: torch.Tensor, qw, epilogue: int, bias: Optional[torch.Tensor]
 def _tracked(t: torch.Tensor) -> bool:
     """Whether something follows operations on ``t`` -- autograd (reverse or
     forward mode), a functorch transform, a dispatch or function mode, a
-    tracer, a tensor subclass: a bias is then added as a separate operation,
-    which it sees."""
-    return ((t.requires_grad and torch.is_grad_enabled())
+    tracer, a tensor subclass -- or its memory holds the values negated: a bias
+    is then added as a separate operation, which sees to that."""
+    return (t.is_neg() or (t.requires_grad and torch.is_grad_enabled())
             or type(t) not in (torch.Tensor, torch.nn.Parameter)
             or getattr(forward_ad, "_current_level", 0) >= 0 or modes_follow())
 

@@ -166,6 +166,7 @@ def _kernel_quantizes(W: torch.Tensor, group_size: int) -> bool:
     operations on it (:func:`modes_follow`)."""
     return (W.is_cuda and W.dtype in _KERNEL_DTYPES and W.numel() > 0
             and type(W) in (torch.Tensor, torch.nn.Parameter) and W.is_contiguous()
+            and not W.is_neg()  # a view whose values are its memory's, negated
             and 8 <= group_size <= _KERNEL_MAX_GROUP and W.shape[0] // group_size < 65536
             and not torch.compiler.is_compiling() and not modes_follow())
 

@@ -255,3 +255,5 @@ def test_bias_under_vmap_and_modes(M, layout):
     assert torch.Tensor.add in seen and torch.equal(watched, y + biases[0])
     with torch.device("cuda"):
         assert not ops._tracked(biases[0])
+    # a view whose memory holds the values negated
+    assert torch.equal(ng.matmul_bias(Xd, qw, torch._neg_view(biases[0])), y - biases[0])

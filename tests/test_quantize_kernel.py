@@ -67,6 +67,10 @@ def test_views_and_other_dtypes_take_the_operations():
         got = ng.quantize_device(V, 64) if V.shape[0] % 64 == 0 else None
         if got is not None:
             assert torch.equal(got.qweight, quant._quantize_ops(V.contiguous().float(), 64).qweight)
+    negated = torch._neg_view(W)  # contiguous; its memory holds -values
+    assert not quant._kernel_quantizes(negated, 64)
+    want = ng.quantize_device(-W, 64)
+    assert torch.equal(ng.quantize_device(negated, 64).qweight, want.qweight)
     offset = torch.randn(128 * 64 + 1, device="cuda")[1:].view(128, 64)  # 4-byte aligned rows
     _same(offset, 128)
 
