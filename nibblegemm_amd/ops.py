@@ -120,7 +120,7 @@ def _check_matmul_inputs(X: torch.Tensor, Wq: torch.Tensor, S: torch.Tensor) -> 
         raise RuntimeError("inputs must be contiguous")
     if X.dim() != 2 or Wq.dim() != 2 or S.dim() != 2:
         raise RuntimeError("expected 2-D inputs")
-    if not (X.device == Wq.device == S.device):
+    if not (X.get_device() == Wq.get_device() == S.get_device()):
         raise RuntimeError("all tensors must live on the same device")
 
 
@@ -396,7 +396,7 @@ def _strip_gemv(X: torch.Tensor, w: StripMajorWeight, epilogue: int,
         raise RuntimeError("strip-major weights must be int32 and scales fp16")
     if not (X.is_contiguous() and Wt.is_contiguous() and St.is_contiguous()):
         raise RuntimeError("inputs must be contiguous")
-    if not (X.device == Wt.device == St.device):
+    if not (X.get_device() == Wt.get_device() == St.get_device()):
         raise RuntimeError("all tensors must live on the same device")
     M, K = X.shape
     if M > DECODE_MAX_M:
@@ -524,8 +524,8 @@ def _tracked(t: torch.Tensor) -> bool:
     forward mode), a functorch transform, a dispatch or function mode, a
     tracer, a tensor subclass -- or its memory holds the values negated: a bias
     is then added as a separate operation, which sees to that."""
-    return (t.is_neg() or (t.requires_grad and torch.is_grad_enabled())
-            or type(t) not in (torch.Tensor, torch.nn.Parameter)
+    return ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
+            or (t.requires_grad and torch.is_grad_enabled()) or t.is_neg()
             or getattr(forward_ad, "_current_level", 0) >= 0 or modes_follow())
 
 
@@ -538,7 +538,8 @@ def matmul_bias(X: torch.Tensor, qw: QuantizedWeight, bias: torch.Tensor) -> tor
     (:func:`_tracked`), run the two ops."""
     _check_2d(X, qw)
     fp16_bias = (bias.dtype == torch.float16 and bias.dim() == 1 and bias.numel() == qw.N
-                 and bias.device == X.device and bias.is_contiguous() and not _tracked(bias))
+                 and bias.is_cuda and bias.get_device() == X.get_device() and bias.is_contiguous()
+                 and not _tracked(bias))
     if isinstance(qw, StripMajorWeight):
         if fp16_bias and X.size(0) <= DECODE_MAX_M:
             return _strip_gemv(X, qw, 1, bias, qw.N)

@@ -142,22 +142,33 @@ _KERNEL_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 _KERNEL_MAX_GROUP = 512
 
 
+def _mode_probes(C):
+    """What :func:`modes_follow` asks, looked up once: it runs in every call
+    with a bias, where the names' lookups took most of its time.  None where
+    this torch lacks one."""
+    try:
+        return (C._functorch.peek_interpreter_stack, C._len_torch_dispatch_stack, C._is_tracing,
+                C._len_torch_function_stack, C._get_function_stack_at)
+    except AttributeError:
+        return None
+
+
+_PROBES = _mode_probes(torch._C)
+
+
 def modes_follow() -> bool:
     """Whether a functorch transform, a dispatch or function mode, or a tracer
     follows torch operations (which would not see a kernel launched beside
     them).  A default device (``torch.set_default_device``) is a function mode
     too, but follows factory calls only.  True also where this torch has no
     such name to ask: operations serve every case."""
-    C = torch._C
-    try:
-        functions = C._len_torch_function_stack()
-        return (C._functorch.peek_interpreter_stack() is not None
-                or C._len_torch_dispatch_stack() > 0
-                or (functions > 0 and any(type(C._get_function_stack_at(i)) is not _DeviceContext
-                                          for i in range(functions)))
-                or torch.jit.is_tracing())
-    except AttributeError:
+    if _PROBES is None:
         return True
+    interpreter, dispatch, tracing, functions, function_at = _PROBES
+    if interpreter() is not None or dispatch() or tracing():
+        return True
+    n = functions()
+    return n > 0 and any(type(function_at(i)) is not _DeviceContext for i in range(n))
 
 
 def _kernel_quantizes(W: torch.Tensor, group_size: int) -> bool:

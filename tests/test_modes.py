@@ -43,10 +43,21 @@ def test_modes_and_transforms_are_noticed():
         assert not ops._tracked(t)
 
 
-@pytest.mark.parametrize("owner,name", [(torch._C._functorch, "peek_interpreter_stack"),
-                                        (torch._C, "_len_torch_dispatch_stack"),
-                                        (torch._C, "_len_torch_function_stack"),
-                                        (torch.autograd.forward_ad, "_current_level")])
-def test_a_torch_without_a_name_composes(monkeypatch, owner, name):
-    monkeypatch.delattr(owner, name)
+@pytest.mark.parametrize("missing", ["_functorch", "_len_torch_dispatch_stack", "_len_torch_function_stack",
+                                     "_is_tracing", "_get_function_stack_at"])
+def test_a_torch_without_a_name_composes(monkeypatch, missing):
+    class Other:
+        def __getattr__(self, name):
+            if name == missing:
+                raise AttributeError(name)
+            return getattr(torch._C, name)
+
+    assert quant._mode_probes(torch._C) is not None
+    assert quant._mode_probes(Other()) is None
+    monkeypatch.setattr(quant, "_PROBES", None)
+    assert ops._tracked(torch.ones(4))
+
+
+def test_a_torch_without_forward_levels_composes(monkeypatch):
+    monkeypatch.delattr(torch.autograd.forward_ad, "_current_level")
     assert ops._tracked(torch.ones(4))
