@@ -35,6 +35,7 @@ constexpr int kAttnMaxChunks = 64;     // chunks a launch uses at most
 constexpr int kAttnOneChunk = 384;     // tokens one workgroup takes alone
 constexpr int kAttnWorkgroups = 256;   // one round of the CUs
 constexpr int64_t kAttnRereadBytes = 80 << 20;  // cache bytes read by all parts together
+constexpr int64_t kAttnLlcBytes = int64_t(256) << 20;  // the last-level cache
 
 // y = fp16(x * r * w) with r = 1 / sqrt(mean(x^2) + eps), in fp32 (the
 // transformers LlamaRMSNorm computes the same in fp32 and rounds x * r to
@@ -474,8 +475,9 @@ int plan_attention(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t max_
   NIBBLE_CHECK(max_seq <= kAttnMaxSeq, "max_seq above %d", kAttnMaxSeq);
   p->qpk = static_cast<int>(qpk);
   const int64_t tokens = pos + 1, room = ceil_div(tokens, kChunk);
+  const int64_t cache_bytes = n_kv * tokens * kHeadDim * 4;
   if (room > 1) {
-    p->counter_bytes = align_up(static_cast<size_t>(n_kv) * 4, 256);
+    p->counter_bytes = align_up(static_cast<size_t>(n_kv) * (qpk == 8 ? 2 : 1) * 4, 256);
     p->workspace_bytes = p->counter_bytes + static_cast<size_t>(n_kv) * room * qpk *
                                                 (kHeadDim + 2) * sizeof(float);
   }
@@ -488,17 +490,51 @@ int plan_attention(int64_t n_heads, int64_t n_kv, int64_t head_dim, int64_t max_
   // (4 x 8 15.7, 1 x 32 16.1), 32768 tokens 2 x 16 30.7 (4 x 16 45).  One chunk
   // up to 384 tokens, which saves the exchange: 129 tokens 4.2 (2 chunks 6.2),
   // 256 5.0 (6.3), 512 7.3 (4 chunks 6.7).
-  const int64_t cache_bytes = n_kv * tokens * kHeadDim * 4;
+  // Workgroups of 8 heads hold one wave a SIMD, so 8 heads make two parts
+  // while the second reading comes from the last-level cache: 64 kv heads, 256
+  // / 1024 tokens 1 part 16.3 / 21.0, 2 parts 10 / 18.
+  // One chunk needs no counters and takes as many parts as keep the grid within
+  // a round, or a round and a half where kv heads on 8 XCDs share the rows in
+  // L2: 40 / 64 kv heads of 8, 384 tokens 4 parts 8.7 / 8.9 (1 part 21); 129 of
+  // 2 1 part 8.6 (2 parts 13.3), 256 of 2 11.4 (13.4).  Where the heads alone
+  // make a round, one chunk goes on to 768 tokens: 64 of 8, 700 tokens 12.5 (3
+  // chunks 14.2), 96 of 4, 385 tokens 9.6 (2 chunks of 1 part 12.9).
+  const bool one_chunk =
+      tokens <= (n_kv * qpk >= kAttnWorkgroups ? 2 * kAttnOneChunk : kAttnOneChunk);
+  const int64_t least = qpk == 8 && cache_bytes <= kAttnLlcBytes ? 2 : 1;
+  const int64_t most = !one_chunk || room == 1 ? 2 * kAttnWorkgroups
+                       : n_kv % 8 == 0         ? kAttnWorkgroups * 3 / 2
+                                               : kAttnWorkgroups;
+  // (Beyond the last-level cache only the padding's worth of counters: 256 kv
+  // heads of 8, 4096 tokens 1 part 172, 2 parts 202.)
+  const int64_t counters = static_cast<int64_t>(
+      least == 2 ? p->counter_bytes / 4 : align_up(static_cast<size_t>(n_kv), 64));
   int64_t parts = qpk;
-  while (parts > 1 && ((parts > 2 && parts * cache_bytes > kAttnRereadBytes) ||
-                       n_kv * parts > 2 * kAttnWorkgroups ||
-                       (room > 1 && n_kv * parts > static_cast<int64_t>(p->counter_bytes / 4))))
+  while (parts > least &&
+         (n_kv * parts > most ||
+          (!one_chunk && ((parts > 2 && parts * cache_bytes > kAttnRereadBytes) ||
+                          n_kv * parts > counters))))
     parts /= 2;
-  const int64_t chunks =
-      tokens <= kAttnOneChunk
-          ? 1
-          : std::min<int64_t>({room, kAttnMaxChunks,
-                               std::max<int64_t>(1, kAttnWorkgroups / (n_kv * parts))});
+  // Chunks: one round of the CUs, two where 8 heads make two parts of more than
+  // a quarter round (two workgroups a CU: 40 kv heads, 4096 tokens 6 chunks
+  // 34.2, 3 38.9).  Above half a round of kv heads and parts, the number up to
+  // 4 that wastes the least of the last round, once a workgroup's share is
+  // worth an exchange: 129 kv heads of 4, 2048 tokens 3 chunks 33.0 (1: 48), of
+  // 2 27.0 (27.9), 1024 tokens of 2 18.2 (16.7); 300 of 1, 2048 tokens 4 chunks
+  // 52.8 (61.8), 512 tokens of 4 26.5 (24.0).
+  const int64_t groups = n_kv * parts, heads = qpk / parts;
+  int64_t chunks = 1;
+  if (!one_chunk && groups <= kAttnWorkgroups / 2) {
+    const bool pairs = qpk == 8 && parts == 2 && groups > kAttnWorkgroups / 4;
+    chunks = kAttnWorkgroups * (pairs ? 2 : 1) / groups;
+  } else if (tokens >= 1024 && tokens * heads >= (groups > kAttnWorkgroups ? 1536 : 4096)) {
+    auto waste = [&](int64_t c) {  // rounds of the CUs over what they hold
+      return static_cast<double>(ceil_div(groups * c, kAttnWorkgroups)) / static_cast<double>(c);
+    };
+    for (int64_t c = 2; c <= 4; ++c)
+      if (waste(c) < 0.999 * waste(chunks)) chunks = c;
+  }
+  chunks = std::min<int64_t>({room, kAttnMaxChunks, chunks});
   const int64_t each = align_up(static_cast<size_t>(ceil_div(tokens, chunks)), kRound);
   p->parts = static_cast<int>(parts);
   p->chunk_tokens = static_cast<int>(each);

@@ -380,11 +380,13 @@ def test_glue_step_graph_replay():
 @pytest.mark.parametrize("n_heads,n_kv,pos", [
     (32, 8, 63), (32, 8, 64), (32, 8, 127), (32, 8, 128), (32, 8, 383), (32, 8, 384), (32, 8, 1030),
     (32, 8, 5200), (64, 8, 2600), (64, 8, 3000), (8, 8, 4095), (2, 2, 9000), (8, 1, 700), (16, 2, 12345),
-    (96, 96, 500), (192, 96, 130), (1024, 256, 400)])
+    (96, 96, 500), (192, 96, 130), (1024, 256, 400),
+    (320, 40, 383), (320, 40, 600), (160, 40, 300), (512, 64, 767), (512, 64, 1000), (264, 33, 800), (384, 96, 400),
+    (516, 129, 2100), (258, 129, 2300), (1032, 129, 384), (300, 300, 1600), (2048, 256, 2200)])
 def test_attention_splits(n_heads, n_kv, pos):
-    """Every split of the work: one chunk up to 384 tokens, chunks cut at and
+    """Every split of the work: one chunk up to 384 or 768 tokens, chunks cut at and
     beside the 64-token rounds, one to eight query heads a workgroup, more
-    (kv head, part) pairs than counters.  Against the float32 reference to one
+    (kv head, part) pairs than counters, more kv heads than half the CUs.  Against the float32 reference to one
     fp16 rounding of the output; repeats and replays give the same bits."""
     max_seq = pos + 3
     qkv, kc, vc = _attn_case(n_heads, n_kv, pos, max_seq, seed=pos + n_heads)
