@@ -98,7 +98,9 @@ def test_gemm_workspace_formula():
     """Batches of M <= 32 run the streaming kernels (split-K workspace as for
     gemv), as do M <= 64 whose one 64-row block fills the CUs in one round
     and M <= 128 whose passes over the weights (one per 32 rows) stay under
-    48 MiB; otherwise tiles, split over K only when the tiles are few."""
+    48 MiB; otherwise there is room for K splits, counted in tiles of 64 or
+    128 rows by 128 columns, only when those are few.  (The direct kernel takes
+    as many of the splits as pay.)"""
     ext = ng.extension()
     assert ext.gemm_workspace_bytes(16, 14336, 4096, 128, 6, None) == (256 + 4 * 16 * 4096 * 4, 256)
     assert ext.gemm_workspace_bytes(32, 4096, 14336, 128, 7, None) == (0, 0)
@@ -106,17 +108,16 @@ def test_gemm_workspace_formula():
     # kernel, 64 strips split 4 ways (256 workgroups), both versions
     assert ext.gemm_workspace_bytes(33, 14336, 4096, 128, 6, None) == (256 + 4 * 33 * 4096 * 4, 256)
     assert ext.gemm_workspace_bytes(33, 14336, 4096, 128, 7, None) == (256 + 4 * 33 * 4096 * 4, 256)
-    # 4096 x 14336: 224 strips unsplit at M = 64 (one block), 224 unsplit
-    # 64-row tiles at M = 128
+    # 4096 x 14336: 224 strips unsplit at M = 64 (one block), 224 tiles of 64
+    # rows at M = 128
     assert ext.gemm_workspace_bytes(64, 4096, 14336, 128, 6, None) == (0, 0)
     assert ext.gemm_workspace_bytes(128, 4096, 14336, 128, 6, None) == (0, 0)
     # 4096 x 4096: one 64-row block at M = 33, its 64 strips split 4 ways;
     # 4096 x 6144 (192 workgroups at most) streams 32-row blocks, unsplit
     assert ext.gemm_workspace_bytes(33, 4096, 4096, 128, 6, None) == (256 + 4 * 33 * 4096 * 4, 256)
     assert ext.gemm_workspace_bytes(33, 4096, 6144, 128, 6, None) == (0, 0)
-    # M > 128 runs the producer/consumer kernel; over a long K (224 steps of
-    # 64) with 128 x 128 tiles split by their count: 2 x 32 = 64 tiles 4 ways
-    # (both versions: the same plan, so the same bits)
+    # M > 128 over a long K (224 steps of 64): 128 x 128 tiles split by their
+    # count, 2 x 32 = 64 tiles 4 ways (both versions)
     assert ext.gemm_workspace_bytes(129, 14336, 4096, 128, 6, None) == (256 + 4 * 129 * 4096 * 4, 256)
     assert ext.gemm_workspace_bytes(129, 14336, 4096, 128, 7, None) == (256 + 4 * 129 * 4096 * 4, 256)
     # 3 x 32 = 96 and 4 x 32 = 128 tiles split 2 ways; 1536 rows (384 tiles,
@@ -131,23 +132,17 @@ def test_gemm_workspace_formula():
     assert ext.gemm_workspace_bytes(129, 4096, 4096, 128, 6, None) == (512 + 4 * 129 * 4096 * 4, 512)
     assert ext.gemm_workspace_bytes(256, 4096, 6144, 128, 6, None) == (0, 0)
     assert ext.gemm_workspace_bytes(129, 4096, 4096, 128, 7, None) == (0, 0)
-    # N % 4 != 0 cannot stream nor take 16-byte B loads: the tile kernel, 33
-    # tiles of 64 x 128, split 4 ways
+    # N % 4 != 0 cannot stream: 33 tiles of 64 x 128, split 4 ways
     assert ext.gemm_workspace_bytes(16, 14336, 4098, 128, 6, None) == (256 + 4 * 16 * 4098 * 4, 256)
     # 192 and 256 tiles of 128 x 128 are not split; above 128 rows a short K
     # never splits
     assert ext.gemm_workspace_bytes(768, 14336, 4096, 128, 6, None) == (0, 0)
     assert ext.gemm_workspace_bytes(1024, 14336, 4096, 128, 7, None) == (0, 0)
     assert ext.gemm_workspace_bytes(512, 4096, 14336, 128, 6, None) == (0, 0)
-    # from M = 1024 version 6 takes 256 x 256 tiles where they make one round
-    # of the CUs (224 tiles here), never split; from M = 2048, 256 x 128
-    # tiles where they make whole rounds (256 at 2048 x 4096), never split
+    # tall batches fill the CUs: never split
     assert ext.gemm_workspace_bytes(1024, 4096, 14336, 128, 6, None) == (0, 0)
     assert ext.gemm_workspace_bytes(2048, 14336, 4096, 128, 6, None) == (0, 0)
-    # 3072 x 4096: 384 such tiles, a round and a half, so 128 x 128 tiles
-    # (768, enough not to split)
     assert ext.gemm_workspace_bytes(3072, 14336, 4096, 128, 6, None) == (0, 0)
-    # version 7 keeps 128 x 128 tiles: 16 x 32 of them at M = 2048, no split
     assert ext.gemm_workspace_bytes(2048, 14336, 4096, 128, 7, None) == (0, 0)
     assert ext.gemm_workspace_bytes(16, 14336, 4096, 128, 5, None) == (0, 0)
 

@@ -276,7 +276,7 @@ def test_gemm_rejects_bad_version():
 @pytest.mark.parametrize("K_,N,g", [(4096, 1024, 128), (14336, 512, 128), (1024, 260, 64)])
 def test_small_batch_handover(M, K_, N, g):
     """M <= 128 runs the weight-streaming kernel (32-row blocks, split over K
-    when K is long), M = 129 the tile kernel; both against the oracle."""
+    when K is long), M = 129 the direct kernel; both against the oracle."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, g, seed=M * 3 + N)
     ref = oracle_y(X, packed, scales, K_, g)
     for version in (6, 7):
@@ -289,10 +289,10 @@ def test_small_batch_handover(M, K_, N, g):
                                     for K_, N in ((4096, 14336), (14336, 4096), (8192, 8192))]
                          + [(100, 14336, 4100), (47, 8192, 8200), (65, 4096, 14340),
                             (40, 4096, 28672), (64, 8192, 14336)])
-def test_small_batch_tiles(M, K_, N):
+def test_small_batches_in_tiles(M, K_, N):
     """Batches of 33..128 rows over large weights (32-row weight passes of
     48 MiB or more, where one 64-row block would not make one round of the
-    CUs) take 64-row producer/consumer tiles split over K instead of
+    CUs) take the direct kernel's tiles, with teams or splits of K, instead of
     streaming: every output, both versions (the same plan, so the same
     bits), repeated calls bit-identical, against an fp32 product of the
     dequant kernel's weights on the GPU.  Three shapes end in partial row
@@ -314,10 +314,11 @@ def test_small_batch_tiles(M, K_, N):
 @pytest.mark.parametrize("M,K_,N", [(129, 4096, 4096), (192, 4096, 4096), (256, 4096, 4096),
                                     (160, 4096, 6144), (200, 6144, 4096), (256, 4096, 6144)])
 def test_mid_k_split(M, K_, N):
-    """4096 <= K < 8192 with at most 160 64-row tiles splits K 4 ways (all
-    but 256 x 4096 x 6144, whose 192 tiles run unsplit; 200 x 6144 x 4096
-    has a row tail and 24 k steps per split): every output against an fp32
-    product of the dequant kernel's weights, repeated calls bit-identical."""
+    """4096 <= K < 8192 with at most 160 tiles of 64 x 128 has room for 4 K
+    splits (all but 256 x 4096 x 6144, with 192 such tiles; 200 x 6144 x 4096
+    has a row tail), of which the plan takes what pays: every output against
+    an fp32 product of the dequant kernel's weights, repeated calls
+    bit-identical."""
     _, _, _, Xd, qw = synthetic(M, K_, N, 128, seed=500 + M + N)
     ref = Xd.float() @ ng.dequant(qw).float()
     rms = ref.pow(2).mean().sqrt()
@@ -330,10 +331,10 @@ def test_mid_k_split(M, K_, N):
 @pytest.mark.parametrize("M,K_,N", [(64, 14336, 4096), (129, 4096, 4096), (160, 14336, 512),
                                     (24, 14336, 1024)])
 def test_split_plans_repeat_their_bits(M, K_, N):
-    """Every split plan's last-arriver sum, called 300 times back to back
-    (64-row tiles split 8 ways, 4096 <= K < 8192 split 4 ways, 128-row tiles
-    split 4 ways, the streaming kernel's split K): identical bits each time,
-    so no call reads a partial before it is complete."""
+    """Shapes with room for K splits -- the batch kernel's 64-row block, 4096
+    <= K < 8192, a long K with few columns, the streaming kernel's split K --
+    called 300 times back to back: identical bits each time, so no call reads
+    a partial before it is complete."""
     _, _, _, Xd, qw = synthetic(M, K_, N, 128, seed=900 + M)
     ext = ng.extension()
     assert ext.gemm_workspace_bytes(M, K_, N, 128, 6, None)[1] > 0  # a split plan
@@ -353,7 +354,7 @@ def test_small_batch_split_k_is_deterministic():
 
 @pytest.mark.parametrize("M,K_,N", [(140, 8192, 640), (200, 14336, 256), (300, 8192, 1024),
                                     (133, 8192, 130)])
-def test_tile_kernel_split_k(M, K_, N):
+def test_few_tiles_split_k(M, K_, N):
     """Few output tiles over a long K split the reduction across workgroups
     (deterministic last-arriver sum); both versions against the oracle."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, 128, seed=M + K_ + N)
@@ -383,10 +384,10 @@ def test_sixteen_row_strip_blocks(M, K_, N, g):
 
 @pytest.mark.parametrize("M,K_,N,g", [(129, 320, 132, 64), (257, 576, 260, 64), (1000, 128, 4100, 128),
                                       (300, 8256, 516, 64), (192, 4096, 640, 128)])
-def test_producer_consumer_kernel_edges(M, K_, N, g):
-    """Shapes for the 64-k producer/consumer kernel: row and column tails of
-    its 64/128-row, 128-column tiles, odd numbers of 64-k steps, group 64 and
-    a K split (K >= 8192)."""
+def test_more_rows_than_stream(M, K_, N, g):
+    """Just past 128 rows and on: row and column tails, odd numbers of 64-k
+    steps, both groups, and a long K over few columns; both versions against
+    the oracle."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
     ref = oracle_y(X, packed, scales, K_, g)
     for version in (6, 7):
@@ -399,13 +400,10 @@ def test_producer_consumer_kernel_edges(M, K_, N, g):
 @pytest.mark.parametrize("M,K_,N,g", [(1024, 256, 14336, 128), (4096, 512, 4096, 64),
                                       (1100, 384, 12000, 128), (2048, 256, 14336, 128),
                                       (1024, 320, 14336, 64), (4000, 256, 4000, 64)])
-def test_large_tile_kernel(M, K_, N, g):
-    """Version 6 runs 256 x 256 tiles from M = 1024 when the grid is one round
-    over the CUs, at least 7/8 full: 224 tiles at 1024 x 14336, 256 at
-    4096 x 4096, and with row and column tails 235 at 1100 x 12000 and 256
-    at 4000 x 4000; 2048 x 14336 (448 tiles) runs the twelve-wave 256 x 128
-    kernel instead.  Every kernel sums each output over k in the same order,
-    so version 6 and version 7 (128 x 128) agree to the bit."""
+def test_wide_grids(M, K_, N, g):
+    """Grids of about a round and more of the CUs over a short K (one team, no
+    split), with row and column tails: every output against the oracle, and
+    version 7, which has the same plan there, gives version 6's bits."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
     y6 = ng.gemm(Xd, qw, version=6)
     y7 = ng.gemm(Xd, qw, version=7)
@@ -418,13 +416,9 @@ def test_large_tile_kernel(M, K_, N, g):
 
 @pytest.mark.parametrize("M,K_,N,g", [(2100, 256, 3500, 128), (2048, 320, 4096, 64),
                                       (2049, 448, 3584, 64)])
-def test_twelve_wave_kernel(M, K_, N, g):
-    """Version 6 runs 256 x 128 tiles with eight consumer waves from M = 2048
-    when that grid makes whole rounds of the CUs (the last at least 7/8 full)
-    and the 256 x 256 kernel does not: with row and column tails (252 tiles
-    at 2100 x 3500), an odd number of 64-k steps with group 64 (256 tiles),
-    and a single-row tail (252 tiles at 2049 x 3584).  Its k order is the
-    128 x 128 kernel's, so version 6 and version 7 agree to the bit."""
+def test_tall_batches(M, K_, N, g):
+    """Batches of 2048 rows and a few more over a short K: row and column
+    tails, an odd number of 64-k steps with group 64, a single-row tail."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
     y6 = ng.gemm(Xd, qw, version=6)
     y7 = ng.gemm(Xd, qw, version=7)
@@ -445,10 +439,9 @@ def _offset_copy(t: torch.Tensor, elems: int) -> torch.Tensor:
 
 @pytest.mark.parametrize("M,K_,N", [(300, 512, 260), (600, 1024, 512)])
 def test_gemm_under_aligned_weights(M, K_, N):
-    """Weights only 8-byte (packed) / 4-byte (scales) aligned cannot take the
-    producer/consumer kernel's 16-byte loads and run the tile kernel; both
-    sum every output over k in the same order, so without a K split the bits
-    agree."""
+    """Weights only 8-byte (packed) / 4-byte (scales) aligned run the direct
+    kernel as aligned ones do: the same bits, and those of the oracle's
+    product to the tolerance."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, 128, seed=M + N)
     qw_off = ng.QuantizedWeight(_offset_copy(qw.qweight, 2), _offset_copy(qw.scales, 2),
                                 qw.group_size, qw.K, qw.N)
@@ -457,6 +450,46 @@ def test_gemm_under_aligned_weights(M, K_, N):
     y_off = ng.gemm(Xd, qw_off)
     assert torch.equal(y, y_off)
     assert rms_err(host(y_off), oracle_y(X, packed, scales, K_, 128)) <= RMS_TOL
+
+
+@pytest.mark.parametrize("words,scale", [(1, 1), (1, 0), (0, 1)])
+@pytest.mark.parametrize("M,K_,N,g", [(9, 128, 2, 64), (33, 320, 66, 64), (65, 192, 258, 64), (16, 1024, 256, 128),
+                                      (129, 64, 130, 64), (300, 448, 260, 64), (600, 1024, 510, 128),
+                                      (2100, 128, 1028, 128), (129, 4096, 512, 128)])
+def test_tile_kernel(M, K_, N, g, words, scale):
+    """Packed words 4-byte or scales 2-byte aligned, which the direct kernel's
+    loads of two columns cannot take, run the tile kernel: both tile heights,
+    row, column and step remainders, both groups, batches and sizes whose
+    aligned call streams or splits K.  Against the oracle; with one team and no
+    split (K below 512, more rows than stream) the direct kernel sums in the
+    same order, so the bits are the aligned call's."""
+    X, packed, scales, Xd, qw = synthetic(M, K_, N, g, seed=M + K_ + N)
+    off = ng.QuantizedWeight(_offset_copy(qw.qweight, words), _offset_copy(qw.scales, scale), g, K_, N)
+    assert off.qweight.data_ptr() % 8 == 4 * words and off.scales.data_ptr() % 4 == 2 * scale
+    ref = oracle_y(X, packed, scales, K_, g)
+    same = K_ < 512 and not ng.extension().gemm_streams(M, K_, N, g)
+    for version in (6, 7):
+        y = ng.gemm(Xd, off, version=version)
+        assert torch.equal(ng.gemm(Xd, off, version=version), y)
+        assert rms_err(host(y), ref) <= RMS_TOL, version
+        if same:
+            assert torch.equal(ng.gemm(Xd, qw, version=version), y), version
+
+
+@pytest.mark.parametrize("M,N", [(40, (1 << 22) + 2), (129, 1 << 22)])
+def test_tile_kernel_widest(M, N):
+    """A width whose tile rows pass the direct kernel's 32-bit offsets."""
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    Wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (8, N), generator=gen, dtype=torch.int32, device="cuda")
+    S = (torch.rand((1, N), generator=gen, device="cuda") * 0.01).half()
+    Xd = torch.randn((M, 64), generator=gen, device="cuda").half()
+    qw = ng.QuantizedWeight(Wq, S, 64, 64, N)
+    y = ng.gemm(Xd, qw)
+    W = ng.dequant(qw)
+    for n in range(0, N, 1 << 20):  # in slices: a float product of 2 GiB and more is beyond torch's
+        ref = Xd.float() @ W[:, n:n + (1 << 20)].float().contiguous()
+        err = (y[:, n:n + (1 << 20)].float() - ref).abs().max()
+        assert float(err / ref.pow(2).mean().sqrt()) <= RMS_TOL
 
 
 @pytest.mark.parametrize("words,scale", [(2, 2), (2, 0), (0, 2)])
@@ -488,11 +521,10 @@ def test_split_plans_under_aligned_weights(M, K_, N, words, scale):
 
 @pytest.mark.parametrize("M,K_,N", [(160, 14336, 512), (64, 14336, 4096), (129, 4096, 4096)])
 def test_split_k_gemm_replays_in_a_graph(M, K_, N):
-    """The producer/consumer kernel's K split (counters reset by the kernel
-    itself, no memset) is graph-capturable; every replay matches eager, with
-    eager work between replays.  Shapes: 128-row tiles split 4 ways over a
-    long K; a small batch on 64-row tiles split 8 ways; 4096 <= K < 8192 with
-    few tiles, split 4 ways."""
+    """K splits (counters reset by the kernel itself, no memset) are
+    graph-capturable; every replay matches eager, with eager work between
+    replays.  Shapes with room for splits: a long K over few columns, the
+    batch kernel's 64-row block, and 4096 <= K < 8192 with few tiles."""
     X, packed, scales, Xd, qw = synthetic(M, K_, N, 128, seed=11)
     ext = ng.extension()
     assert ext.gemm_workspace_bytes(M, K_, N, 128, 6, None)[1] > 0  # this plan splits K
