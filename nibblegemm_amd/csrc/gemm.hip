@@ -72,26 +72,13 @@ struct TileCfg {
   static constexpr int VB = BN / 64;                // packed words per thread per step
   static_assert(TM >= 1 && TN >= 1, "wave tile must hold a 32 x 32 MFMA tile");
   static_assert(A_ITERS >= 1, "A tile must give every thread a chunk");
-  static_assert(VB == 1 || VB == 2 || VB == 4, "B words per thread");
+  static_assert(VB == 1 || VB == 2, "B words per thread");
 };
 
 // VB adjacent packed words (and their fp16 scales) of one packed row, as one
 // buffer load each.
 template <int VB>
 struct BWords;
-template <>
-struct BWords<4> {
-  using word_t = u4_t;
-  using scale_t = h4_t;
-  static __device__ __forceinline__ word_t load_w(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-    return __builtin_bit_cast(u4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
-  }
-  static __device__ __forceinline__ scale_t load_s(__amdgpu_buffer_rsrc_t r, uint32_t v, uint32_t s) {
-    return __builtin_bit_cast(h4_t, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0));
-  }
-  static __device__ __forceinline__ uint32_t word(word_t w, int j) { return w[j]; }
-  static __device__ __forceinline__ _Float16 scale(scale_t x, int j) { return x[j]; }
-};
 template <>
 struct BWords<2> {
   using word_t = u2_t;
@@ -124,82 +111,9 @@ struct TileArgs {
   const uint32_t* Wq;
   const _Float16* S;
   _Float16* Y;
-  float* partial;      // [splits, M, N] fp32 when splits > 1
-  uint32_t* counters;  // [tiles], zero on entry and on exit
   int M, K, N;
-  int steps_per_split;  // 32-k steps per K split
-  int splits;
-  WeightLayout L;       // where a column's words and scales live (packed or strip-major)
+  WeightLayout L;  // where a column's words and scales live (packed or strip-major)
 };
-
-// Last-arriver sum of a split output tile [m0, m0 + BM) x [n0, n0 + BN) by
-// the whole workgroup: each thread takes 16-byte chunks of 4 columns and
-// loads the chunk's partial of every split (up to 4 in one round, with the
-// same device-coherent cache policy as load_coherent) before adding them in
-// split order, then stores the 4 fp16 results.  Chunks go two at a time, so
-// a thread has at most 8 loads in flight and the kernels keep their
-// register budget.  Needs N % 4 == 0 (16-byte partial rows, 8-byte output
-// stores) and M * N * 4 < 2^31 (32-bit buffer offsets; the plans split only
-// grids of a few hundred tiles).
-template <int THREADS, int BM, int BN>
-__device__ __forceinline__ void tile_sum_splits(const TileArgs& args, int m0, int n0) {
-  constexpr int QUADS = BN / 4;
-  constexpr int CHUNKS = BM * QUADS;
-  constexpr int kPair = 2, kBatch = 4;
-  constexpr bool kWholeRounds = CHUNKS % (THREADS * kPair) == 0;
-  constexpr uint32_t kCoherent = 16;  // sc1: the cache policy of an agent-scope load
-  const int M = args.M, N = args.N;
-  const uint32_t plane = static_cast<uint32_t>(M) * static_cast<uint32_t>(N);
-  // The ABI asks only 2-byte alignment of Y: 8-byte stores when it has more.
-  const bool y_quads = (reinterpret_cast<uintptr_t>(args.Y) & 7u) == 0;
-#pragma nounroll
-  for (int c0 = 0; c0 < CHUNKS; c0 += THREADS * kPair) {
-    uint32_t off[kPair];
-    bool ok[kPair];
-#pragma unroll
-    for (int u = 0; u < kPair; ++u) {
-      const int c = c0 + u * THREADS + static_cast<int>(threadIdx.x);
-      const int gm = m0 + c / QUADS, gn = n0 + 4 * (c % QUADS);
-      ok[u] = gm < M && gn < N && (kWholeRounds || c < CHUNKS);
-      off[u] = ok[u] ? (static_cast<uint32_t>(gm) * N + gn) * 4u : kOutOfRange;
-    }
-    f4_t sum[kPair] = {};
-    for (int sp0 = 0; sp0 < args.splits; sp0 += kBatch) {
-      f4_t v[kBatch][kPair];
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b) {
-        const int sp = sp0 + b < args.splits ? sp0 + b : 0;
-        const __amdgpu_buffer_rsrc_t rp =
-            make_rsrc(args.partial + static_cast<size_t>(sp) * plane, plane * 4u);
-#pragma unroll
-        for (int u = 0; u < kPair; ++u)
-          v[b][u] = __builtin_bit_cast(
-              f4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, off[u], 0, kCoherent));
-      }
-#pragma unroll
-      for (int b = 0; b < kBatch; ++b)
-        if (sp0 + b < args.splits) {
-#pragma unroll
-          for (int u = 0; u < kPair; ++u)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum[u][e] += v[b][u][e];
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < kPair; ++u)
-      if (ok[u]) {
-        const h4_t y = {(_Float16)sum[u][0], (_Float16)sum[u][1], (_Float16)sum[u][2],
-                        (_Float16)sum[u][3]};
-        _Float16* dst = args.Y + off[u] / 4;
-        if (y_quads) {
-          *reinterpret_cast<h4_t*>(dst) = y;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dst[e] = y[e];
-        }
-      }
-  }
-}
 
 template <int BM, int BN, int GROUP>
 __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1, 2))) void
@@ -208,7 +122,6 @@ gemm_tile_kernel(TileArgs args) {
   constexpr int VB = C::VB;
   __shared__ __attribute__((aligned(16))) _Float16 As[2][BM * LDK];
   __shared__ __attribute__((aligned(16))) _Float16 Bs[2][BN * LDK];
-  __shared__ int s_last;
   const _Float16* __restrict__ X = args.X;
   const uint32_t* __restrict__ Wq = args.Wq;
   const _Float16* __restrict__ S = args.S;
@@ -248,9 +161,7 @@ gemm_tile_kernel(TileArgs args) {
   // n0 + VB * (tid % 64) .. + VB - 1.
   const int b_row = tid >> 6;
   const int b_col = n0 + VB * (tid & 63);
-  // This workgroup's K split: steps [step0, step0 + ntiles) of 32 k.
-  const int step0 = blockIdx.z * args.steps_per_split;
-  const int ntiles = min(args.steps_per_split, K / BK - step0);
+  const int ntiles = K / BK;
   const uint32_t row_bytes = args.L.w_row;
   const __amdgpu_buffer_rsrc_t rx =
       make_rsrc(X, static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 2u);
@@ -273,7 +184,7 @@ gemm_tile_kernel(TileArgs args) {
   // re-reads it (an L2 hit) rather than being skipped, so the loads are the
   // same on every path and the compiler's in-order wait counts stay exact.
   auto load_step = [&](Stage& st, int step) {
-    const uint32_t k0 = static_cast<uint32_t>((step0 + min(step, ntiles - 1)) * BK);
+    const uint32_t k0 = static_cast<uint32_t>(min(step, ntiles - 1) * BK);
 #pragma unroll
     for (int it = 0; it < C::A_ITERS; ++it)
       st.a[it] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(rx, voff_a[it], k0 * 2u, 0));
@@ -360,29 +271,8 @@ gemm_tile_kernel(TileArgs args) {
   // Epilogue: register r of lane l holds row 8*(r/4) + 4*(l/32) + r%4,
   // column l % 32 of each 32 x 32 tile.
   const int rq = (lane >> 5) * 4;
-  if (args.splits == 1) {
 #pragma unroll
-    for (int i = 0; i < C::TM; ++i) {
-#pragma unroll
-      for (int j = 0; j < C::TN; ++j) {
-        const int gn = n0 + wn + 32 * j + r32;
-        if (gn >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gm = m0 + wm + 32 * i + 8 * (r >> 2) + rq + (r & 3);
-          if (gm < M) Y[static_cast<size_t>(gm) * N + gn] = (_Float16)acc[i][j][r];
-        }
-      }
-    }
-    return;
-  }
-
-  // K split: publish this split's fp32 tile with device-coherent stores; the
-  // last workgroup of the tile (agent-scope counter) sums the splits in
-  // split order and writes Y -- deterministic, one launch.
-  float* part = args.partial + static_cast<size_t>(blockIdx.z) * M * N;
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i)
+  for (int i = 0; i < C::TM; ++i) {
 #pragma unroll
     for (int j = 0; j < C::TN; ++j) {
       const int gn = n0 + wn + 32 * j + r32;
@@ -390,44 +280,10 @@ gemm_tile_kernel(TileArgs args) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int gm = m0 + wm + 32 * i + 8 * (r >> 2) + rq + (r & 3);
-        if (gm < M) store_coherent(part + static_cast<size_t>(gm) * N + gn, acc[i][j][r]);
+        if (gm < M) Y[static_cast<size_t>(gm) * N + gn] = (_Float16)acc[i][j][r];
       }
     }
-  // Last-arriver exchange; relies on gfx950 hardware ordering: see
-  // "HARDWARE ASSUMPTION" in nibble_decode.h.
-  wait_vm_stores();
-  __syncthreads();
-  const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-  if (tid == 0) {
-    const uint32_t prev =
-        __hip_atomic_fetch_add(args.counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == static_cast<uint32_t>(args.splits - 1));
   }
-  __syncthreads();
-  if (!s_last) return;
-  if (N % 4 == 0) {
-    tile_sum_splits<kGemmThreads, BM, BN>(args, m0, n0);
-  } else {
-#pragma unroll
-    for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < C::TN; ++j) {
-        const int gn = n0 + wn + 32 * j + r32;
-        if (gn >= N) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int gm = m0 + wm + 32 * i + 8 * (r >> 2) + rq + (r & 3);
-          if (gm >= M) continue;
-          const size_t off = static_cast<size_t>(gm) * N + gn;
-          float sum = 0.0f;
-          for (int sp = 0; sp < args.splits; ++sp)
-            sum += load_coherent(args.partial + static_cast<size_t>(sp) * M * N + off);
-          Y[off] = (_Float16)sum;
-        }
-      }
-  }
-  if (tid == 0)
-    __hip_atomic_store(args.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int TM, int KW, int WN>
@@ -447,8 +303,7 @@ hipError_t launch_direct_cfg(DirectArgs a, int64_t G, hipStream_t stream) {
 
 template <int BM, int BN>
 hipError_t launch_tile(const TileArgs& a, int64_t G, hipStream_t stream) {
-  dim3 grid(static_cast<unsigned>(ceil_div(a.N, BN)), static_cast<unsigned>(ceil_div(a.M, BM)),
-            static_cast<unsigned>(a.splits));
+  dim3 grid(static_cast<unsigned>(ceil_div(a.N, BN)), static_cast<unsigned>(ceil_div(a.M, BM)));
   if (G == 128)
     gemm_tile_kernel<BM, BN, 128><<<grid, kGemmThreads, 0, stream>>>(a);
   else
@@ -470,9 +325,6 @@ constexpr int kPlanCUs = 256;
 // The widest B vector aligned operands of this N allow (the plan the
 // workspace query assumes).
 int nominal_bn_max(int64_t N) { return N % 4 == 0 ? 256 : N % 2 == 0 ? 128 : 64; }
-
-// k per pipeline step of the kernel a choice runs.
-int step_k(TileChoice t) { return t.tm > 0 ? kDirectStep : BK; }
 
 // Widest B vector (BN / 64 packed words per thread) the operands allow.
 int max_bn(int64_t N, const void* w, const void* s) {
@@ -498,7 +350,6 @@ TileChoice choose_tile(int64_t M, int64_t N, int bn_max) {
 struct TilePlan {
   TileChoice t;
   int splits = 1;
-  int steps_per_split = 0;
   size_t counter_bytes = 0;
   size_t workspace_bytes = 0;
 };
@@ -542,7 +393,6 @@ TilePlan plan_split_room(int64_t M, int64_t K, int64_t N, int64_t version, int b
       splits = static_cast<int>(std::min<int64_t>(ceil_div(2 * kPlanCUs, tiles), 4));
   }
   const int64_t steps = K / unit, per = ceil_div(steps, splits);
-  p.steps_per_split = static_cast<int>(per * (unit / BK));
   p.splits = static_cast<int>(ceil_div(steps, per));
   if (p.splits > 1) {
     p.counter_bytes = align_up(static_cast<size_t>(tiles) * 4, 256);
@@ -642,20 +492,19 @@ TileChoice choose_direct(int64_t M, int64_t K, int64_t N, const TilePlan& room, 
   return best;
 }
 
-// The launch plan.  `direct` says the operands suit the direct kernel, which
-// loads two columns at a time whatever more their alignment allows (bn_max):
-// its room is the workspace query's, so the splits, the workspace they need
-// and where the counters end are what the caller was told.  Both versions
-// take the same plan wherever their workspaces agree, and then agree to the
-// bit.
+// The launch plan.  The direct kernel (`direct`: the operands suit it) loads
+// two columns at a time whatever more their alignment allows (bn_max): its
+// room is the workspace query's, so the splits, the workspace they need and
+// where the counters end are what the caller was told.  The tile kernel never
+// splits K: it runs only under-aligned operands, or an N whose K is short.
+// The versions' plans differ only where the room does (version 7 has none for
+// 4096 <= K < 8192, and other splits where N % 4 == 2); elsewhere they are the
+// same, with the same bits.
 TilePlan plan_tile(int64_t M, int64_t K, int64_t N, int64_t version, int bn_max, bool direct) {
   TilePlan p = plan_split_room(M, K, N, version, direct ? nominal_bn_max(N) : bn_max);
-  if (direct) {
-    int splits = 1;
-    p.t = choose_direct(M, K, N, p, &splits);
-    p.splits = splits;
-    p.steps_per_split = static_cast<int>(ceil_div(K / kDirectStep, splits));
-  }
+  int splits = 1;
+  if (direct) p.t = choose_direct(M, K, N, p, &splits);
+  p.splits = splits;
   return p;
 }
 
@@ -834,25 +683,14 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
   // tall activations are run in row blocks that stay below 2^31 bytes (such
   // grids are far too large to need a K split).
   const int64_t rows_max = std::max<int64_t>(256, ((int64_t(1) << 31) - 1) / (K * 2) / 256 * 256);
-  // The workspace query plans for aligned operands; when the pointers force
-  // another kernel than that plan's (tiles where the query planned the
-  // streaming kernel, or another tile), the call runs without a split, as do
-  // row-blocked tall launches.
-  const bool nominal_direct = direct_supported(K, N, nullptr, nullptr);
-  const TilePlan nominal = bn_max == nominal_bn_max(N) && direct == nominal_direct
-                               ? p
-                               : plan_tile(M, K, N, version, nominal_bn_max(N), nominal_direct);
-  if (M > rows_max || gemm_streams(M, K, N, group_size) || p.t.tm != nominal.t.tm ||
-      p.t.kw != nominal.t.kw || p.t.bm != nominal.t.bm || p.t.bn != nominal.t.bn ||
-      p.splits != nominal.splits)
-    p.splits = 1;
+  // Row-blocked tall launches run without a split, as do small batches whose
+  // pointers rule out the streaming kernel that the workspace query planned.
+  if (M > rows_max || gemm_streams(M, K, N, group_size)) p.splits = 1;
   if (p.splits > 1) {
     if (workspace == nullptr || workspace_bytes < p.workspace_bytes)
       return fail(NIBBLE_ERR_WORKSPACE, "gemm needs %zu bytes of workspace, got %zu",
                   p.workspace_bytes, workspace == nullptr ? size_t(0) : workspace_bytes);
     if (!aligned(workspace, 256)) return fail(NIBBLE_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  } else {
-    p.steps_per_split = static_cast<int>(K / step_k(p.t));
   }
   auto* counters = p.splits > 1 ? static_cast<uint32_t*>(workspace) : nullptr;
   auto* partial = p.splits > 1
@@ -876,7 +714,7 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
       a.K = static_cast<int>(K);
       a.N = static_cast<int>(N);
       a.splits = p.splits;
-      a.steps_per_split = p.steps_per_split;
+      a.steps_per_split = static_cast<int>(ceil_div(K / kDirectStep, p.splits));
       a.epilogue = epilogue;
       a.L = layout;
       e = launch_direct(p.t, a, group_size, stream);
@@ -887,13 +725,9 @@ int gemm_run(const void* X, int64_t M, int64_t K, int64_t N, const void* Wq, con
     a.Wq = static_cast<const uint32_t*>(Wq);
     a.S = static_cast<const _Float16*>(S);
     a.Y = y + m0 * N;
-    a.partial = partial;
-    a.counters = counters;
     a.M = rows;
     a.K = static_cast<int>(K);
     a.N = static_cast<int>(N);
-    a.steps_per_split = p.steps_per_split;
-    a.splits = p.splits;
     a.L = layout;
     e = launch_choice(p.t, a, group_size, stream);
   }
