@@ -151,8 +151,10 @@ NIBBLE_API int nibble_gemv_timeline(void* stamps, int64_t bytes);
 
 /*
  * Prefill-regime matmul on CDNA4 MFMA (any M >= 1).  version 6 (default) or 7
- * (same numerics).  Requires K % 32 == 0, N even,
- * group_size in {64, 128} and M*N, M*K, K*N < 2^31 (the reference's checks).
+ * (the same arithmetic; some sizes have room for K splits in version 6 alone
+ * or for others in version 7, whose sums then round differently).  Requires
+ * K % 32 == 0, N even, group_size in {64, 128} and M*N, M*K, K*N < 2^31 (the
+ * reference's checks).
  * Small batches (with N % 4 == 0) run the weight-streaming kernels of the
  * GEMV where nibble_gemm_streams says so, larger ones tiles; either may split
  * K across workgroups.  `workspace` follows the same rules as for nibble_gemv_w4a16,
@@ -196,7 +198,6 @@ NIBBLE_API int nibble_gemm_w4a16_fused(const void* X, int64_t x_rows, int64_t x_
                         int64_t group_size, int64_t strip_cols, int64_t epilogue,
                         const void* bias, void* Y, void* workspace,
                         size_t workspace_bytes, void* stream);
-
 
 /*
  * Streaming matmul (1 <= M <= 128) with a fused output epilogue.  No

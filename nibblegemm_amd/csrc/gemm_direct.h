@@ -353,7 +353,8 @@ __global__ __launch_bounds__(KW* WN * 64, OCC) void gemm_direct_kernel(DirectArg
   Words R[RING];
   // Part p (a quarter) of the copies of a step, and of its words: slice p's,
   // with part 0 the scales.  Steps past the last read through empty resources
-  // (no access), so every wave's count of loads in flight stays exact.
+  // (no access: gfx950's range check takes the scalar offset in without
+  // wrapping), so every wave's count of loads in flight stays exact.
   auto copy_part = [&](auto pc, int step, int buf) {
     constexpr int p = decltype(pc)::value;
     constexpr int c0 = p * COPIES / 4, c1 = (p + 1) * COPIES / 4;

@@ -284,9 +284,11 @@ def gemv(X: torch.Tensor, qw: QuantizedWeight, version: int = 4, splits: int = 0
 
 def gemm(X: torch.Tensor, qw: QuantizedWeight, version: int = 6) -> torch.Tensor:
     """Prefill-regime matmul on MFMA (reference ops.py:77-86).  ``version`` 6
-    (default) or 7, with identical numerics: the plan depends on the sizes
-    only.  Small batches run the GEMV's weight-streaming kernels (up to 32
-    rows, and up to 128 over weights small enough), larger ones tiles.  A
+    (default) or 7: the same arithmetic, on a plan that depends on the sizes
+    and the version (some sizes have room for K splits in one only, whose sums
+    then round differently).  Small batches run the GEMV's weight-streaming
+    kernels (up to 32 rows, and up to 128 over weights small enough), larger
+    ones tiles.  A
     :class:`StripMajorWeight` runs the same plans and kernels (the same bits
     as its packed weight) from 9 rows, the strip-major GEMV below."""
     if isinstance(qw, StripMajorWeight):
@@ -319,7 +321,7 @@ def to_strip_major(qw: QuantizedWeight, strip_cols: int = 0) -> StripMajorWeight
     (one permutation kernel on the current stream; same bytes again).
     ``strip_cols`` 0 picks :func:`strip_major_cols`.  The result serves
     :func:`matmul`, :func:`gemm`, :func:`dequant` and the fused ops at every
-    batch size (the fused epilogues run in the kernel up to 8 rows)."""
+    batch size."""
     ext = _bind()
     Wq, S = qw.qweight, qw.scales
     if not (Wq.is_cuda and S.is_cuda):
@@ -417,8 +419,8 @@ def _strip_gemv(X: torch.Tensor, w: StripMajorWeight, epilogue: int,
 
 def matmul(X: torch.Tensor, qw, splits: int = 0, block_threads: int = 0) -> torch.Tensor:
     """``X @ dequant(qw)``, dispatching on batch size (reference ops.py:89-104):
-    M <= DECODE_MAX_M goes to ``gemv(version=4)``, larger M to ``gemm``.  A
-    :class:`StripMajorWeight` (M <= 8 only) runs the strip-major GEMV."""
+    M <= DECODE_MAX_M goes to ``gemv(version=4)``, larger M to ``gemm``; on a
+    :class:`StripMajorWeight` to the strip-major GEMV and the same GEMM."""
     if X.dim() != 2:
         raise ValueError(f"expected a 2-D activation matrix, got {tuple(X.shape)}")
     if X.size(1) != qw.K:
@@ -448,10 +450,9 @@ def _fused_workspace(ext, device: torch.device, stream: int, M: int, K: int, N: 
 
 def _fusable(X: torch.Tensor, qw: QuantizedWeight) -> bool:
     """Whether the fused-epilogue launch takes these operands and computes
-    the product with ``matmul``'s bits (else the caller composes the same
-    arithmetic from separate ops).  The fused launch streams; ``matmul``
-    takes tiles for batches of 33..128 rows over large weights, so those
-    compose."""
+    the product with ``matmul``'s bits.  The fused launch streams; ``matmul``
+    takes tiles for batches of 33..128 rows over large weights
+    (:func:`_gemm_fusable`)."""
     return (X.dim() == 2 and X.is_cuda and 1 <= X.size(0) <= FUSED_MAX_M and qw.N % 4 == 0
             and X.is_contiguous() and X.data_ptr() % 16 == 0
             and qw.qweight.data_ptr() % 16 == 0 and qw.scales.data_ptr() % 8 == 0

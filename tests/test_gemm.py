@@ -493,7 +493,7 @@ def test_tile_kernel_widest(M, N):
 
 
 @pytest.mark.parametrize("words,scale", [(2, 2), (2, 0), (0, 2)])
-@pytest.mark.parametrize("M,K_,N", [(96, 8192, 8192), (384, 14336, 4096), (129, 8192, 4096)])
+@pytest.mark.parametrize("M,K_,N", [(96, 8192, 8192), (128, 8192, 8192), (256, 14336, 4096)])
 def test_split_plans_under_aligned_weights(M, K_, N, words, scale):
     """Weights 8-byte and scales 4-byte aligned run the aligned call's plan with
     its K splits, in the workspace that the query reports: the same bits."""
