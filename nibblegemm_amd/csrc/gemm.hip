@@ -587,8 +587,10 @@ namespace {
 // kernel's tiles win (plan_tile).  Measured, graph replay, streaming against
 // tiles: 4096 x 14336 M = 65 / 128 25 / 41.9 us against 17.2 / 19.0; 14336 x
 // 4096 M = 128 56.6 against 23.6; 8192 x 8192 M = 96 43 against 23.2.  Below
-// that streaming stays ahead or level: 4096 x 4096 M = 33..128 10.6-12.6 us
-// against 12.9-14.0, 4096 x 6144 M = 64 12.7 against 14.0.
+// that streaming was ahead or level when the line was drawn; the tiles of one
+// column wave have come level with it since, and ahead from 65 rows: 4096 x
+// 4096 M = 64 / 128 10.9 / 11.9 us against 11.6 / 11.6, 4096 x 6144 M = 64 / 65
+// / 96 11.7 / 16.3 / 21.0 against 11.3 / 14.6 / 14.7.
 bool gemm_streams(int64_t M, int64_t K, int64_t N, int64_t G) {
   if (!(M >= 1 && M <= kStreamMaxM && K > 0 && N > 0 && N % 4 == 0 && K % G == 0)) return false;
   const int64_t pass_bytes = K * N / 2;
