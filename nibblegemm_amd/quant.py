@@ -140,6 +140,7 @@ def quantize(W: torch.Tensor, group_size: int = 128, clip_search: bool = False) 
 #: Weight dtypes the quantisation kernel reads, and its largest group.
 _KERNEL_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 _KERNEL_MAX_GROUP = 512
+_get_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _mode_probes(C):
@@ -196,10 +197,16 @@ def quantize_device(W: torch.Tensor, group_size: int = 128) -> QuantizedWeight:
         ext = _native.binding()
         packed = torch.empty((K // PACK_FACTOR, N), dtype=torch.int32, device=W.device)
         scales = torch.empty((K // group_size, N), dtype=torch.float16, device=W.device)
-        with torch.cuda.device(W.device):  # a null stream is the current device's
-            rc = ext.quantize_rtn(W.data_ptr(), K, N, _KERNEL_DTYPES[W.dtype], group_size,
-                                  packed.data_ptr(), scales.data_ptr(),
-                                  torch.cuda.current_stream(W.device).cuda_stream)
+        index = W.get_device()
+        stream = (torch.cuda.current_stream(index).cuda_stream if _get_raw_stream is None
+                  else _get_raw_stream(index))
+        args = (W.data_ptr(), K, N, _KERNEL_DTYPES[W.dtype], group_size, packed.data_ptr(),
+                scales.data_ptr(), stream)
+        if index == torch.cuda.current_device():
+            rc = ext.quantize_rtn(*args)
+        else:  # a null stream is the current device's
+            with torch.cuda.device(W.device):
+                rc = ext.quantize_rtn(*args)
         if rc:
             raise RuntimeError(f"nibblegemm_amd: {ext.last_error()} (status {rc})")
         return QuantizedWeight(packed, scales, group_size, K, N)

@@ -208,13 +208,13 @@ def test_quantize_device_launches_on_the_weights_device(monkeypatch):
             launched.append((list(current), args[1:5]))
             return 0
 
-    class Null:
-        cuda_stream = 0
-
     monkeypatch.setattr(quant, "_kernel_quantizes", lambda W, g: True)
     monkeypatch.setattr(_native, "binding", lambda: Stub)
     monkeypatch.setattr(torch.cuda, "device", device)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: Null)
+    monkeypatch.setattr(quant, "_get_raw_stream", lambda index: 0)
     W = torch.randn(128, 16)
-    quant.quantize_device(W, 64)
-    assert launched == [([W.device], (128, 16, 2, 64))] and not current
+    for index, entered in ((0, [W.device]), (W.get_device(), [])):  # another device, W's own
+        monkeypatch.setattr(torch.cuda, "current_device", lambda index=index: index)
+        launched.clear()
+        quant.quantize_device(W, 64)
+        assert launched == [(entered, (128, 16, 2, 64))] and not current
